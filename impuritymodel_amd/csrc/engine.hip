@@ -872,6 +872,7 @@ KrylovBatch krylov_view(Batch* b) {
                  b->val.as<double2>(),
                  b->h_n,
                  b->h_nnz};
+  kb.real = b->real;
   bool flat = false;
   for (int c = 0; c < b->C; ++c) flat = flat || b->h_n[c] > g_tuning.flat_min_n;
   if (b->real && flat && g_tuning.real_values) {

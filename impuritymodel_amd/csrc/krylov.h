@@ -19,6 +19,7 @@ struct KrylovBatch {
   // the real parts of val when every value is real (NULL otherwise): the
   // grid-wide SpMV then reads 8 bytes per value instead of 16
   const double* val_re = nullptr;
+  bool real = false;  // every value is real
 };
 
 // Plain (reorth = 0) or fully reorthogonalized (reorth = 1) Lanczos from v0

@@ -22,6 +22,7 @@
 #include <mutex>
 
 #include "krylov.h"
+#include "krylov_reg.h"
 
 namespace imped {
 
@@ -94,24 +95,6 @@ template <int BT, class T>
 __device__ void dots_lds(const T* V, int m, int64_t n, const T* w, double2* cl, bool self);
 template <int BT, class T>
 __device__ double update_norm(const T* V, int m, int64_t n, T* w, const double2* cl, double* red);
-
-struct LanczosArgs {
-  const int64_t* row_base;
-  const int64_t* chain_n;
-  const int64_t* rowptr;
-  const int32_t* col;
-  const double2* val;
-  const double2* v0;
-  int K;
-  int reorth;
-  double2* ws;      // 3 vectors per chain at 3*row_base
-  double2* vstore;  // reorth: K vectors per chain at K*row_base (coefficients in LDS)
-  double* alpha;
-  double* beta;
-  int32_t* kout;
-  int32_t* status;
-  const int32_t* chain_list;  // chains handled by this launch, one per workgroup
-};
 
 template <int BT>
 __global__ __launch_bounds__(BT) void lanczos_kernel(LanczosArgs a) {
@@ -188,483 +171,9 @@ __global__ __launch_bounds__(BT) void lanczos_kernel(LanczosArgs a) {
   }
 }
 
-// ---- fully reorthogonalized Lanczos with the Krylov basis in LDS
-//
-// For a chain whose K' = min(K, n) Krylov vectors fit in LDS next to the
-// residual, one wave runs the whole recurrence on LDS: V[l] at row l of
-// stride s (the smallest s >= n with s = 1 mod 8, so both the row-parallel
-// update, lane i reading V[l][i], and the vector-parallel dot pass, lane l
-// reading V[l][i], touch 64 distinct LDS banks), then w, then the
-// Gram-Schmidt coefficients.  The dot pass gives lane l the whole product
-// <V_l, w> (a sequential sum over rows), so a step needs no per-vector
-// wave reductions.  The SpMV, alpha, beta and three-term update are those
-// of lanczos_kernel; v_{j-1} and v_j are rows j-1 and j of V.
-
+// Row stride of an LDS-held basis: the smallest s >= n with s = 1 mod 8, so
+// accesses along rows and along vectors both spread over the banks.
 __device__ __forceinline__ int64_t lds_row_stride(int64_t n) { return (n + 6) / 8 * 8 + 1; }
-
-size_t lanczos_lds_bytes(int64_t n, int K) {
-  const int64_t kk = K < n ? K : n;
-  const int64_t s = (n + 6) / 8 * 8 + 1;
-  return (size_t)(kk * s + s + kk + 2) * sizeof(double2);
-}
-
-__global__ __launch_bounds__(64) void lanczos_lds_kernel(LanczosArgs a) {
-  extern __shared__ double2 lds[];
-  const int c = a.chain_list[blockIdx.x];
-  const int64_t n = a.chain_n[c];
-  const int64_t base = a.row_base[c];
-  double* alpha = a.alpha + (size_t)c * a.K;
-  double* beta = a.beta + (size_t)c * a.K;
-  const int lane = threadIdx.x;
-  if (n == 0) {
-    if (lane == 0) {
-      a.kout[c] = 0;
-      a.status[c] = IMPED_OK;
-    }
-    return;
-  }
-  const int K = (int)(a.K < n ? a.K : n);
-  const int64_t s = lds_row_stride(n);
-  double2* V = lds;
-  double2* w = V + (size_t)K * s;
-  double2* cl = w + s;
-  const int64_t* rowptr = a.rowptr + base;
-  // The first row of every lane (row = lane) keeps up to RC of its entries
-  // in registers for all K steps, so most of the SpMV reads no memory; the
-  // rest of the row, and rows from 64 on, are read from memory each step.
-  constexpr int RC = 16;
-  double2 hv[RC];
-  int hc[RC];
-  int64_t r0e1 = 0, r0rest = 0;
-  int hn = 0;
-  if (lane < n) {
-    const int64_t e0 = rowptr[lane];
-    r0e1 = rowptr[lane + 1];
-    hn = (int)(r0e1 - e0 < RC ? r0e1 - e0 : RC);
-    r0rest = e0 + hn;
-#pragma unroll
-    for (int k = 0; k < RC; ++k) {
-      hv[k] = k < hn ? a.val[e0 + k] : make_double2(0.0, 0.0);
-      hc[k] = k < hn ? a.col[e0 + k] : 0;
-    }
-  }
-  // y = H x and Re<x, y> over the chain's rows (x, y in LDS)
-  auto spmv = [&](const double2* x, double2* y) {
-    double pa = 0.0;
-    if (lane < n) {
-      double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
-#pragma unroll
-      for (int k = 0; k < RC; k += 2) {
-        if (k < hn) {
-          const double2 v = x[hc[k]];
-          ax += hv[k].x * v.x - hv[k].y * v.y;
-          ay += hv[k].x * v.y + hv[k].y * v.x;
-        }
-        if (k + 1 < hn) {
-          const double2 v = x[hc[k + 1]];
-          bx += hv[k + 1].x * v.x - hv[k + 1].y * v.y;
-          by += hv[k + 1].x * v.y + hv[k + 1].y * v.x;
-        }
-      }
-      for (int64_t e = r0rest; e < r0e1; ++e) {
-        const double2 h = a.val[e];
-        const double2 v = x[a.col[e]];
-        ax += h.x * v.x - h.y * v.y;
-        ay += h.x * v.y + h.y * v.x;
-      }
-      ax += bx;
-      ay += by;
-      y[lane] = make_double2(ax, ay);
-      pa += ax * x[lane].x + ay * x[lane].y;
-    }
-    for (int64_t i = lane + 64; i < n; i += 64) {
-      const int64_t e0 = rowptr[i], e1 = rowptr[i + 1];
-      double ax = 0.0, ay = 0.0;
-      for (int64_t e = e0; e < e1; ++e) {
-        const double2 h = a.val[e];
-        const double2 v = x[a.col[e]];
-        ax += h.x * v.x - h.y * v.y;
-        ay += h.x * v.y + h.y * v.x;
-      }
-      y[i] = make_double2(ax, ay);
-      pa += ax * x[i].x + ay * x[i].y;
-    }
-    return wave_sum(pa);
-  };
-  // one classical Gram-Schmidt pass against V_0..V_{m-1}; returns |w|^2.
-  // Two partial sums per product (even and odd terms) halve the dependent
-  // chain of additions.
-  auto gram_schmidt = [&](int m) {
-    for (int l = lane; l < m; l += 64) {
-      const double2* vl = V + (size_t)l * s;
-      double cx = 0.0, cy = 0.0, dx = 0.0, dy = 0.0;
-      int64_t i = 0;
-#pragma unroll 2
-      for (; i + 1 < n; i += 2) {
-        const double2 v = vl[i], b = w[i], v1 = vl[i + 1], b1 = w[i + 1];
-        cx += v.x * b.x + v.y * b.y;
-        cy += v.x * b.y - v.y * b.x;
-        dx += v1.x * b1.x + v1.y * b1.y;
-        dy += v1.x * b1.y - v1.y * b1.x;
-      }
-      if (i < n) {
-        const double2 v = vl[i], b = w[i];
-        cx += v.x * b.x + v.y * b.y;
-        cy += v.x * b.y - v.y * b.x;
-      }
-      cl[l] = make_double2(cx + dx, cy + dy);
-    }
-    __syncthreads();
-    double p = 0.0;
-    for (int64_t i = lane; i < n; i += 64) {
-      double ux = 0.0, uy = 0.0, tx = 0.0, ty = 0.0;
-      int l = 0;
-#pragma unroll 4
-      for (; l + 1 < m; l += 2) {
-        const double2 cc = cl[l], c1 = cl[l + 1];
-        const double2 av = V[(size_t)l * s + i], a1 = V[(size_t)(l + 1) * s + i];
-        ux += av.x * cc.x - av.y * cc.y;
-        uy += av.x * cc.y + av.y * cc.x;
-        tx += a1.x * c1.x - a1.y * c1.y;
-        ty += a1.x * c1.y + a1.y * c1.x;
-      }
-      if (l < m) {
-        const double2 cc = cl[l];
-        const double2 av = V[(size_t)l * s + i];
-        ux += av.x * cc.x - av.y * cc.y;
-        uy += av.x * cc.y + av.y * cc.x;
-      }
-      const double wx = w[i].x - (ux + tx), wy = w[i].y - (uy + ty);
-      w[i] = make_double2(wx, wy);
-      p += wx * wx + wy * wy;
-    }
-    __syncthreads();
-    return wave_sum(p);
-  };
-  for (int64_t i = lane; i < n; i += 64) V[i] = a.v0[base + i];
-  __syncthreads();
-  // wp = H v0; alpha0 = Re(conj(wp) . v0); w = wp - alpha0 v0
-  double al = spmv(V, w);
-  if (lane == 0) alpha[0] = al;
-  for (int64_t i = lane; i < n; i += 64) w[i] = make_double2(w[i].x - al * V[i].x, w[i].y - al * V[i].y);
-  __syncthreads();
-  int status = IMPED_OK;
-  int kdone = K;
-  for (int j = 1; j < K; ++j) {
-    double p = 0.0;
-    for (int64_t i = lane; i < n; i += 64) p += w[i].x * w[i].x + w[i].y * w[i].y;
-    p = wave_sum(p);
-    // full reorthogonalization against V_0..V_{j-1}; a second pass when
-    // the first removed more than half of |w|^2 (as lanczos_kernel)
-    double p1 = gram_schmidt(j);
-    if (p1 < 0.5 * p) p1 = gram_schmidt(j);
-    const double b = sqrt(p1);
-    if (lane == 0) beta[j - 1] = b;
-    if (b == 0.0) {
-      status = IMPED_ERR_BREAKDOWN;
-      kdone = j;
-      break;
-    }
-    double2* vj = V + (size_t)j * s;
-    const double2* vp = vj - s;
-    for (int64_t i = lane; i < n; i += 64) vj[i] = make_double2(w[i].x / b, w[i].y / b);
-    __syncthreads();
-    al = spmv(vj, w);
-    if (lane == 0) alpha[j] = al;
-    for (int64_t i = lane; i < n; i += 64) {
-      const double2 x = vj[i], y = vp[i];
-      w[i] = make_double2(w[i].x - al * x.x - b * y.x, w[i].y - al * x.y - b * y.y);
-    }
-    __syncthreads();
-  }
-  if (lane == 0) {
-    a.kout[c] = kdone;
-    a.status[c] = status;
-  }
-}
-
-// ---- the same recurrence with NW waves per chain
-//
-// lanczos_lds_kernel leaves each step's Gram-Schmidt products as one long
-// sequential sum per lane (n terms for a dot, m for an update) on a single
-// wave.  Here NW waves share a chain: for the dots, wave g sums rows
-// [g n/NW, (g+1) n/NW) of every <V_l, w> (lane l); for the update, wave g
-// sums vectors [g m/NW, (g+1) m/NW) of every row (lane), each lane adding
-// the NW dot partials of the coefficients it needs itself; the NW update
-// partials of each row are then subtracted from w.  Each dependent chain is
-// NW times shorter and the chain's CU runs NW times as many waves.  Row t
-// of the SpMV (t < 64 NW) keeps up to RC entries of H in registers.
-//
-// The update is owned by rows: wave g updates rows [g n/NW, (g+1) n/NW) of
-// w (the rows whose dot partials it formed), each row on a quad of lanes
-// that splits the vectors (lane q takes l = q, q + 4, ...; DPP adds the
-// quad), with the coefficients added from the NW dot partials once per wave
-// into a row of its own.  A step takes four workgroup barriers: the SpMV
-// reads w scaled by 1/beta (so no pass writes v_j before it) into a second
-// residual buffer, |w|^2 is posted by the three-term update and summed
-// after the next barrier, and a Gram-Schmidt pass needs one barrier after
-// its dots and one for the sum of |w|^2.  LDS: V (K rows of stride s), w,
-// w2, NW x K dot partials and NW x K coefficients.
-
-size_t lanczos_ldsw_bytes(int64_t n, int K, int nw) {
-  const int64_t kk = K < n ? K : n;
-  const int64_t s = (n + 6) / 8 * 8 + 1;
-  return (size_t)(kk * s + 2 * s + 2 * nw * kk) * sizeof(double2);
-}
-
-template <int NW>
-__global__ __launch_bounds__(64 * NW) void lanczos_ldsw_kernel(LanczosArgs a) {
-  constexpr int T = 64 * NW;
-  constexpr int RC = 16;
-  extern __shared__ double2 lds[];
-  __shared__ double red[2][NW];
-  const int c = a.chain_list[blockIdx.x];
-  const int64_t n = a.chain_n[c];
-  const int64_t base = a.row_base[c];
-  double* alpha = a.alpha + (size_t)c * a.K;
-  double* beta = a.beta + (size_t)c * a.K;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  if (n == 0) {
-    if (tid == 0) {
-      a.kout[c] = 0;
-      a.status[c] = IMPED_OK;
-    }
-    return;
-  }
-  const int K = (int)(a.K < n ? a.K : n);
-  const int64_t s = lds_row_stride(n);
-  double2* V = lds;
-  double2* w = V + (size_t)K * s;
-  double2* w2 = w + s;
-  double2* dotp = w2 + s;                 // [NW][K]
-  double2* coefw = dotp + (size_t)NW * K;  // [NW][K], a row per wave
-  const int64_t* rowptr = a.rowptr + base;
-  // workgroup sums: post() leaves each wave's partial in a row of red
-  // (rows used in turn), collect() adds them after a barrier; a row is
-  // written again only two posts later, past a barrier that follows every
-  // collect of it
-  int rsel = 0;
-  auto post = [&](double x) {
-    x = wave_sum(x);
-    if (lane == 0) red[rsel][wv] = x;
-    const int r = rsel;
-    rsel ^= 1;
-    return r;
-  };
-  auto collect = [&](int r) {
-    double t = 0.0;
-#pragma unroll
-    for (int g = 0; g < NW; ++g) t += red[r][g];
-    return t;
-  };
-  // a row of H on tpr = 4, 2 or 1 threads (as many as n rows leave room
-  // for): thread tid takes row tid / tpr and holds up to RC of its entries
-  // tid % tpr, tid % tpr + tpr, ... in registers; DPP adds the row's lanes
-  const int tpr = 4 * n <= T ? 4 : (2 * n <= T ? 2 : 1);
-  const int64_t hrow = tid / tpr;
-  double2 hv[RC];
-  int hc[RC];
-  int64_t r_end = 0, r_rest = 0;
-  int hn = 0;
-  if (hrow < n) {
-    const int64_t e0 = rowptr[hrow] + tid % tpr;
-    r_end = rowptr[hrow + 1];
-    const int64_t mine = r_end > e0 ? (r_end - e0 + tpr - 1) / tpr : 0;
-    hn = (int)(mine < RC ? mine : RC);
-    r_rest = e0 + (int64_t)hn * tpr;
-#pragma unroll
-    for (int k = 0; k < RC; ++k) {
-      hv[k] = k < hn ? a.val[e0 + (int64_t)k * tpr] : make_double2(0.0, 0.0);
-      hc[k] = k < hn ? a.col[e0 + (int64_t)k * tpr] : 0;
-    }
-  }
-  // the wave's longest register share: groups of four entries past it are
-  // skipped (a wave-uniform branch); inside a group every load is issued
-  // unconditionally (entries past a row's end hold 0 at column 0)
-  const int hn_wave = wave_max_int(hn);
-  // y = H (sc x) over the rows of this thread, and its part of Re<sc x, y>;
-  // xj (when not null) receives sc x for those rows
-  auto spmv = [&](const double2* x, double sc, double2* y, double2* xj) {
-    double pa = 0.0;
-    double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
-    if (hrow < n) {
-#pragma unroll
-      for (int k0 = 0; k0 < RC; k0 += 4) {
-        if (k0 < hn_wave) {
-          double2 v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] = x[hc[k0 + u]];
-#pragma unroll
-          for (int u = 0; u < 4; u += 2) {
-            ax += hv[k0 + u].x * v[u].x - hv[k0 + u].y * v[u].y;
-            ay += hv[k0 + u].x * v[u].y + hv[k0 + u].y * v[u].x;
-            bx += hv[k0 + u + 1].x * v[u + 1].x - hv[k0 + u + 1].y * v[u + 1].y;
-            by += hv[k0 + u + 1].x * v[u + 1].y + hv[k0 + u + 1].y * v[u + 1].x;
-          }
-        }
-      }
-      for (int64_t e = r_rest; e < r_end; e += tpr) {
-        const double2 h = a.val[e];
-        const double2 v = x[a.col[e]];
-        ax += h.x * v.x - h.y * v.y;
-        ay += h.x * v.y + h.y * v.x;
-      }
-    }
-    ax = row_lanes_sum(ax + bx, tpr) * sc;
-    ay = row_lanes_sum(ay + by, tpr) * sc;
-    if (hrow < n && tid % tpr == 0) {
-      y[hrow] = make_double2(ax, ay);
-      const double2 xi = make_double2(x[hrow].x * sc, x[hrow].y * sc);
-      if (xj) xj[hrow] = xi;
-      pa += ax * xi.x + ay * xi.y;
-    }
-    for (int64_t i = tid + T; i < n; i += T) {
-      const int64_t e0 = rowptr[i], e1 = rowptr[i + 1];
-      double ax = 0.0, ay = 0.0;
-      for (int64_t e = e0; e < e1; ++e) {
-        const double2 h = a.val[e];
-        const double2 v = x[a.col[e]];
-        ax += h.x * v.x - h.y * v.y;
-        ay += h.x * v.y + h.y * v.x;
-      }
-      ax *= sc;
-      ay *= sc;
-      y[i] = make_double2(ax, ay);
-      const double2 xi = make_double2(x[i].x * sc, x[i].y * sc);
-      if (xj) xj[i] = xi;
-      pa += ax * xi.x + ay * xi.y;
-    }
-    return pa;
-  };
-  // one classical Gram-Schmidt pass of w against V_0..V_{m-1} (w complete
-  // on entry); returns |w|^2 and leaves w complete
-  auto gram_schmidt = [&](int m) {
-    const int64_t r0 = n * wv / NW, r1 = n * (wv + 1) / NW;
-    for (int l = lane; l < m; l += 64) {
-      const double2* vl = V + (size_t)l * s;
-      double cx = 0.0, cy = 0.0, dx = 0.0, dy = 0.0;
-      int64_t i = r0;
-#pragma unroll 4
-      for (; i + 1 < r1; i += 2) {
-        const double2 v = vl[i], b = w[i], v1 = vl[i + 1], b1 = w[i + 1];
-        cx += v.x * b.x + v.y * b.y;
-        cy += v.x * b.y - v.y * b.x;
-        dx += v1.x * b1.x + v1.y * b1.y;
-        dy += v1.x * b1.y - v1.y * b1.x;
-      }
-      if (i < r1) {
-        const double2 v = vl[i], b = w[i];
-        cx += v.x * b.x + v.y * b.y;
-        cy += v.x * b.y - v.y * b.x;
-      }
-      dotp[(size_t)wv * K + l] = make_double2(cx + dx, cy + dy);
-    }
-    __syncthreads();
-    // the coefficients, added from the NW dot partials by each wave into its
-    // own row (read back by the same wave only, after its own writes)
-    double2* cw = coefw + (size_t)wv * K;
-    for (int l = lane; l < m; l += 64) {
-      double2 t = dotp[l];
-#pragma unroll
-      for (int g = 1; g < NW; ++g) {
-        const double2 u = dotp[(size_t)g * K + l];
-        t.x += u.x;
-        t.y += u.y;
-      }
-      cw[l] = t;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const int q = lane & 3;
-    double p = 0.0;
-    for (int64_t rb = r0; rb < r1; rb += 16) {
-      const int64_t i = rb + (lane >> 2);
-      const bool on = i < r1;
-      const int64_t ii = on ? i : r0;  // idle lanes read a valid row, their sums are dropped
-      double ux = 0.0, uy = 0.0, tx = 0.0, ty = 0.0;
-      int l = q;
-#pragma unroll 2
-      for (; l + 4 < m; l += 8) {
-        const double2 c0 = cw[l], c1 = cw[l + 4];
-        const double2 v0 = V[(size_t)l * s + ii], v1 = V[(size_t)(l + 4) * s + ii];
-        ux += v0.x * c0.x - v0.y * c0.y;
-        uy += v0.x * c0.y + v0.y * c0.x;
-        tx += v1.x * c1.x - v1.y * c1.y;
-        ty += v1.x * c1.y + v1.y * c1.x;
-      }
-      if (l < m) {
-        const double2 c0 = cw[l];
-        const double2 v0 = V[(size_t)l * s + ii];
-        ux += v0.x * c0.x - v0.y * c0.y;
-        uy += v0.x * c0.y + v0.y * c0.x;
-      }
-      ux += tx;
-      uy += ty;
-      ux += dpp_move<0xB1, 0xF>(ux);  // quad_perm [1,0,3,2]
-      uy += dpp_move<0xB1, 0xF>(uy);
-      ux += dpp_move<0x4E, 0xF>(ux);  // quad_perm [2,3,0,1]
-      uy += dpp_move<0x4E, 0xF>(uy);
-      if (on && q == 0) {
-        const double wx = w[i].x - ux, wy = w[i].y - uy;
-        w[i] = make_double2(wx, wy);
-        p += wx * wx + wy * wy;
-      }
-    }
-    const int r = post(p);
-    __syncthreads();
-    return collect(r);
-  };
-  for (int64_t i = tid; i < n; i += T) V[i] = a.v0[base + i];
-  __syncthreads();
-  // w2 = H v0; alpha0 = Re(conj(w2) . v0); w = w2 - alpha0 v0
-  int r = post(spmv(V, 1.0, w2, nullptr));
-  __syncthreads();
-  double al = collect(r);
-  if (tid == 0) alpha[0] = al;
-  double p = 0.0;
-  for (int64_t i = tid; i < n; i += T) {
-    const double wx = w2[i].x - al * V[i].x, wy = w2[i].y - al * V[i].y;
-    w[i] = make_double2(wx, wy);
-    p += wx * wx + wy * wy;
-  }
-  int rp = post(p);
-  __syncthreads();
-  int status = IMPED_OK;
-  int kdone = K;
-  for (int j = 1; j < K; ++j) {
-    const double pw = collect(rp);
-    // full reorthogonalization against V_0..V_{j-1}; a second pass when
-    // the first removed more than half of |w|^2 (as lanczos_kernel)
-    double p1 = gram_schmidt(j);
-    if (p1 < 0.5 * pw) p1 = gram_schmidt(j);
-    const double b = sqrt(p1);
-    if (tid == 0) beta[j - 1] = b;
-    if (b == 0.0) {
-      status = IMPED_ERR_BREAKDOWN;
-      kdone = j;
-      break;
-    }
-    double2* vj = V + (size_t)j * s;
-    const double2* vp = vj - s;
-    // v_j = w / beta is formed inside the SpMV (rows by their owners)
-    r = post(spmv(w, 1.0 / b, w2, vj));
-    __syncthreads();
-    al = collect(r);
-    if (tid == 0) alpha[j] = al;
-    p = 0.0;
-    for (int64_t i = tid; i < n; i += T) {
-      const double2 x = vj[i], y = vp[i];
-      const double wx = w2[i].x - al * x.x - b * y.x, wy = w2[i].y - al * x.y - b * y.y;
-      w[i] = make_double2(wx, wy);
-      p += wx * wx + wy * wy;
-    }
-    rp = post(p);
-    __syncthreads();
-  }
-  if (tid == 0) {
-    a.kout[c] = kdone;
-    a.status[c] = status;
-  }
-}
 
 // ------------------------------------------------------------------ eigen
 
@@ -2799,7 +2308,7 @@ struct KScratch {
   DevBuf ws, vstore, coef, ab, yk, tw, tpiv, voff, conv, wbuf, clist;
   DevBuf cf_alpha_tmp, cf_in, gout, sout;
   DevBuf fpart, fcpart, fcoef, fscal;
-  DevBuf sz, scz, sres, ssteps, eig_in;
+  DevBuf sz, scz, sres, ssteps, eig_in, pure;
 };
 KScratch& kscratch() {
   static KScratch k;
@@ -3163,44 +2672,45 @@ int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_
 
 namespace {
 
-// LDS of one chain of lanczos_lds_kernel: two chains per CU (160 KiB).
-constexpr size_t LDS_CHAIN_BYTES = 80 * 1024;
-
-int lds_waves() {
-  const int64_t w = g_tuning.lanczos_lds_waves;
-  return w == 2 || w == 4 ? (int)w : 1;
+// Compute units of the current device (one device per process).
+int device_cus() {
+  static const int n = [] {
+    int v = 0;
+    HIP_CHECK(hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, 0));
+    return v;
+  }();
+  return n;
 }
 
-// LDS of one chain of the LDS-resident Lanczos for the current wave count
-size_t lds_chain_bytes(int64_t n, int K) {
-  const int nw = lds_waves();
-  return nw == 1 ? lanczos_lds_bytes(n, K) : lanczos_ldsw_bytes(n, K, nw);
-}
-
-template <class F>
-void set_lds_limit(F* kernel) {
-  HIP_CHECK(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)LDS_CHAIN_BYTES));
-}
-
-// nb chains (a.chain_list) on the LDS-resident Lanczos, `bytes` of LDS each
-void launch_lanczos_lds(const LanczosArgs& a, unsigned nb, size_t bytes, hipStream_t s) {
-  static std::once_flag once;
-  std::call_once(once, [] {
-    set_lds_limit(lanczos_lds_kernel);
-    set_lds_limit(lanczos_ldsw_kernel<2>);
-    set_lds_limit(lanczos_ldsw_kernel<4>);
-  });
-  switch (lds_waves()) {
-    case 4:
-      hipLaunchKernelGGL(lanczos_ldsw_kernel<4>, dim3(nb), dim3(256), bytes, s, a);
-      break;
-    case 2:
-      hipLaunchKernelGGL(lanczos_ldsw_kernel<2>, dim3(nb), dim3(128), bytes, s, a);
-      break;
-    default:
-      hipLaunchKernelGGL(lanczos_lds_kernel, dim3(nb), dim3(64), bytes, s, a);
+// 1 for a chain whose start vector is real, 2 for a purely imaginary one (both
+// for a zero one), else 0: one wave per chain.
+__global__ __launch_bounds__(64) void pure_start_kernel(const int64_t* row_base, const int64_t* chain_n,
+                                                        const double2* v0, int32_t* pure) {
+  const int c = blockIdx.x;
+  const int64_t n = chain_n[c], base = row_base[c];
+  bool re = true, im = true;
+  for (int64_t i = threadIdx.x; i < n; i += 64) {
+    const double2 t = v0[base + i];
+    re = re && t.y == 0.0;
+    im = im && t.x == 0.0;
   }
+  const bool all_re = __all(re), all_im = __all(im);
+  if (threadIdx.x == 0) pure[c] = all_re ? 1 : (all_im ? 2 : 0);
+}
+
+// The chains of one class (a.chain_list, a.nmax rows at most) on the register
+// kernels.  Groups of waves per chain: as many as the chip's two waves per
+// SIMD hold for all chains at once (a chain's steps are a dependent sequence, so
+// its waves shorten it; past that they only add barriers), at most
+// lanczos_lds_waves.
+void launch_lanczos_reg(const LanczosArgs& a, unsigned nb, hipStream_t s) {
+  const int n_cu = device_cus();
+  const int64_t nq = std::min<int64_t>((a.nmax + 63) / 64, 4);
+  int groups = 4;
+  while (groups > 1 && (groups > g_tuning.lanczos_lds_waves || (int64_t)nb * nq * groups > 8 * (int64_t)n_cu))
+    groups /= 2;
+  if (a.pure) launch_lanczos_reg_real(a, nb, n_cu, groups, s);
+  launch_lanczos_reg_cplx(a, nb, n_cu, groups, s);
 }
 
 }  // namespace
@@ -3233,12 +2743,14 @@ void run_lanczos(const KrylovBatch& kb, const double2* v0, int K, int reorth, do
   a.kout = kout;
   a.status = status;
   if (kb.C == 0) return;
-  // chains bucketed by dimension: with reorthogonalization, chains whose
-  // Krylov basis fits LDS_CHAIN_BYTES get one wave with the basis in LDS;
-  // otherwise one wave, 256 or 1024 threads per chain; the largest (plain
-  // recurrence) run grid-wide, one chain at a time
-  std::vector<int32_t> lists[5], flat;
-  size_t lds_max = 0, house_max = 0;
+  // chains bucketed by dimension: with reorthogonalization, up to kRegMaxN
+  // rows on the register kernels (buckets 4.. by class); otherwise one wave,
+  // 256 or 1024 threads per chain; the largest (plain recurrence) run
+  // grid-wide, one chain at a time
+  constexpr int kBuckets = 4 + kRegClasses;
+  std::vector<int32_t> lists[kBuckets], flat;
+  size_t house_max = 0;
+  int64_t reg_max[kRegClasses] = {};
   const int64_t house_lim = std::min<int64_t>(g_tuning.lanczos_dense_max_n, kDenseMaxN);
   for (int c = 0; c < kb.C; ++c) {
     const int64_t n = kb.h_n[c];
@@ -3247,13 +2759,14 @@ void run_lanczos(const KrylovBatch& kb, const double2* v0, int K, int reorth, do
       continue;
     }
     if (reorth && n <= house_lim) {
-      lists[4].push_back(c);
+      lists[3].push_back(c);
       house_max = std::max(house_max, house_lanczos_bytes(n));
       continue;
     }
-    if (reorth && g_tuning.lanczos_lds && lds_chain_bytes(n, K) <= LDS_CHAIN_BYTES) {
-      lists[3].push_back(c);
-      lds_max = std::max(lds_max, lds_chain_bytes(n, K));
+    if (reorth && g_tuning.lanczos_lds && lanczos_reg_fits(n, K)) {
+      const int k = lanczos_reg_class(n);
+      lists[4 + k].push_back(c);
+      reg_max[k] = std::max(reg_max[k], n);
       continue;
     }
     const int bkt = n <= g_tuning.lanczos_wave_max_n ? 0 : (n <= g_tuning.lanczos_wg256_max_n ? 1 : 2);
@@ -3264,8 +2777,17 @@ void run_lanczos(const KrylovBatch& kb, const double2* v0, int K, int reorth, do
   std::vector<int32_t> all;
   for (auto& l : lists) all.insert(all.end(), l.begin(), l.end());
   h2d(sc.clist, all.data(), all.size(), s);
+  bool reg = false;
+  for (int k = 0; k < kRegClasses; ++k) reg = reg || !lists[4 + k].empty();
+  if (reg && kb.real) {
+    sc.pure.reserve((size_t)kb.C * 4);
+    hipLaunchKernelGGL(pure_start_kernel, dim3(kb.C), dim3(64), 0, s, kb.row_base, kb.chain_n, v0,
+                       sc.pure.as<int32_t>());
+    HIP_CHECK(hipGetLastError());
+    a.pure = sc.pure.as<int32_t>();
+  }
   size_t off = 0;
-  for (int bkt = 0; bkt < 5; ++bkt) {
+  for (int bkt = 0; bkt < kBuckets; ++bkt) {
     const unsigned nb = (unsigned)lists[bkt].size();
     if (!nb) continue;
     a.chain_list = sc.clist.as<int32_t>() + off;
@@ -3277,15 +2799,16 @@ void run_lanczos(const KrylovBatch& kb, const double2* v0, int K, int reorth, do
       hipLaunchKernelGGL(lanczos_kernel<256>, dim3(nb), dim3(256), shm, s, a);
     else if (bkt == 2)
       hipLaunchKernelGGL(lanczos_kernel<1024>, dim3(nb), dim3(1024), shm, s, a);
-    else if (bkt == 3)
-      launch_lanczos_lds(a, nb, lds_max, s);
-    else {
+    else if (bkt == 3) {
       static std::once_flag once;
       std::call_once(once, [] {
         HIP_CHECK(hipFuncSetAttribute((const void*)house_lanczos_kernel<256>,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
       });
       hipLaunchKernelGGL(house_lanczos_kernel<256>, dim3(nb), dim3(256), house_max, s, a);
+    } else {
+      a.nmax = (int)reg_max[bkt - 4];
+      launch_lanczos_reg(a, nb, s);
     }
     HIP_CHECK(hipGetLastError());
   }
@@ -3394,8 +2917,7 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
   const size_t esz = real ? 8 : 16;
   // LDS per workgroup: the whole 160 KiB when every chain of the launch gets
   // its own CU, shared out when several must sit on one CU at once
-  static int n_cu = 0;
-  if (!n_cu) HIP_CHECK(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, 0));
+  const int n_cu = device_cus();
   auto layout = [&](size_t first, int bt, size_t n_chains) {
     const int64_t nmax = kb.h_n[order[first]];
     const int L = (int)std::min<int64_t>(max_steps, nmax);
@@ -3733,9 +3255,10 @@ extern "C" int imped_lanczos_noalloc(const int64_t* rowptr, const int32_t* col, 
     const size_t shm = reorth ? (size_t)(K + 2) * sizeof(double2) : 0;
     // the size buckets of run_lanczos, so a chain gets the same kernel (and
     // the same arithmetic) as through imped_batch_lanczos
-    if (reorth && g_tuning.lanczos_lds && lds_chain_bytes(n, K) <= LDS_CHAIN_BYTES)
-      launch_lanczos_lds(a, 1, lds_chain_bytes(n, K), s);
-    else if (n <= g_tuning.lanczos_wave_max_n)
+    if (reorth && g_tuning.lanczos_lds && lanczos_reg_fits(n, K)) {
+      a.nmax = (int)n;
+      launch_lanczos_reg(a, 1, s);
+    } else if (n <= g_tuning.lanczos_wave_max_n)
       hipLaunchKernelGGL(lanczos_kernel<64>, dim3(1), dim3(64), shm, s, a);
     else if (n <= g_tuning.lanczos_wg256_max_n)
       hipLaunchKernelGGL(lanczos_kernel<256>, dim3(1), dim3(256), shm, s, a);

@@ -86,10 +86,11 @@ int imped_timing_query(const char* name, double* total_ms, int64_t* launches);
  * prediction's kernels run as one replayed HIP graph, which shortens the
  * GPU's span but costs the calling thread more than the launches it
  * replaces; 0, the default: direct launches, as with switched-on timing),
- * "lanczos_lds" (1, the default: a fully reorthogonalized chain whose Krylov
- * basis fits 80 KiB runs on one workgroup with the basis in LDS; 0: the
- * basis in memory), "lanczos_lds_waves" (waves of that workgroup: 1, 2 or
- * 4, the default; the Gram-Schmidt sums are split over the waves). */
+ * "lanczos_lds" (1, the default: a fully reorthogonalized chain of up to
+ * 1024 rows runs on one workgroup with the basis in registers, then LDS,
+ * then memory; 0: the basis in memory), "lanczos_lds_waves" (cap on the
+ * groups of waves of that workgroup, one group holding every row once: 1, 2 or
+ * 4, the default; the basis vectors are split over the groups). */
 int imped_set_tuning(const char* name, int64_t value);
 
 /* The engine's device radix sort (the one that orders BFS layers and

@@ -1,0 +1,102 @@
+"""Register-resident Lanczos (reorth = 1, chains of up to 1024 rows) against a
+numpy recurrence with two Gram-Schmidt passes per step, at the edges of its
+launch classes (64-row steps, one to four rows per thread), with bases that fit
+the registers, that reach into LDS and that reach into memory, for complex,
+real and imaginary start vectors and with enough chains to change the number of
+waves per chain.
+
+Tolerance: the two recurrences differ by rounding only; full
+reorthogonalization keeps the amplification of a step's rounding (about
+eps |H| sqrt(n) = 1e-13 here) at the level of the step count, so 1e-10 of |H|
+leaves more than a factor of four at 200 steps.
+"""
+
+import numpy as np
+import pytest
+import scipy.sparse
+
+pytestmark = pytest.mark.gpu
+
+
+def _lanczos(h, v, K):
+    V, alpha, beta = [v], [], []
+    w = h @ v
+    for j in range(min(K, len(v))):
+        alpha.append(np.vdot(w, V[-1]).real)
+        if j + 1 == min(K, len(v)):
+            break
+        w = w - alpha[-1] * V[-1] - (beta[-1] * V[-2] if j else 0.0)
+        for _ in range(2):
+            m = np.array(V)
+            w = w - m.T @ (m.conj() @ w)
+        beta.append(np.linalg.norm(w))
+        V.append(w / beta[-1])
+        w = h @ V[-1]
+    return np.array(alpha), np.array(beta)
+
+
+def _chain(rng, n, complex_h, start):
+    def part():
+        return scipy.sparse.random(n, n, density=min(1.0, 5.0 / n), random_state=rng,
+                                   data_rvs=lambda k: rng.standard_normal(k)).toarray()
+
+    a = part() + (1j * part() if complex_h else 0.0)
+    h = a + a.conj().T + np.diag(3.0 * rng.standard_normal(n))
+    v = rng.standard_normal(n) + (1j * rng.standard_normal(n) if start == "complex" else 0.0)
+    v = 1j * v if start == "imaginary" else v
+    return scipy.sparse.csr_matrix(h.astype(complex)), v / np.linalg.norm(v)
+
+
+def _run(chains, K):
+    from impuritymodel_amd.engine import Batch, Ops
+
+    b = Batch(Ops([{}], [None], 1), np.zeros(len(chains), np.int32))
+    rowptr = [0]
+    for h, _ in chains:
+        rowptr.extend((h.indptr[1:] + rowptr[-1]).tolist())
+    b.set_csr([h.shape[0] for h, _ in chains], np.array(rowptr, np.int64),
+              np.concatenate([h.indices for h, _ in chains]).astype(np.int32),
+              np.concatenate([h.data for h, _ in chains]))
+    return b.lanczos(K, reorth=1, v0=np.concatenate([v for _, v in chains]))
+
+
+@pytest.mark.parametrize("complex_h,start", [(True, "complex"), (False, "complex"), (False, "real"),
+                                             (False, "imaginary")])
+@pytest.mark.parametrize("sizes,K,copies", [
+    ([1, 2, 3, 36, 37, 63, 64], 64, 1),     # one wave of rows, many waves per chain
+    ([60, 64], 64, 600),                    # one wave per chain, basis in registers and LDS
+    ([65, 128], 128, 1),
+    ([97, 128], 128, 150),
+    ([129, 192], 192, 1),
+    ([193, 256], 150, 2),
+    ([257, 512], 90, 1),                    # two rows per thread, basis into memory
+    ([513, 768], 60, 1),
+    ([769, 1024], 50, 1),
+    ([1024], 200, 1),
+])
+def test_register_lanczos_matches_numpy(gpu, complex_h, start, sizes, K, copies):
+    rng = np.random.default_rng(5)
+    chains = [_chain(rng, n, complex_h, start) for n in sizes]
+    alpha, beta, kout, status = _run(chains * copies, K)
+    for i, (h, v) in enumerate(chains):
+        a, b = _lanczos(h, v, K)
+        scale = max(1.0, abs(h).sum(axis=1).max())
+        for c in range(i, len(chains) * copies, len(chains)):
+            assert (kout[c], status[c]) == (min(K, len(v)), 0)
+            assert np.abs(alpha[c, : len(a)] - a).max() <= 1e-10 * scale
+            assert np.abs(beta[c, : len(b)] - b).max(initial=0.0) <= 1e-10 * scale
+
+
+def test_register_lanczos_breakdown_and_empty_chain(gpu):
+    # an eigenvector of a diagonal H as start vector: beta_0 is exactly zero
+    from impuritymodel_amd._lib import IMPED_ERR_BREAKDOWN
+
+    h = scipy.sparse.diags(np.arange(1.0, 6.0)).tocsr().astype(complex)
+    e = np.zeros(5, complex)
+    e[2] = 1.0
+    rng = np.random.default_rng(6)
+    other = _chain(rng, 70, True, "complex")
+    alpha, _, kout, status = _run([(h, e), other, (scipy.sparse.csr_matrix((0, 0), dtype=complex), e[:0])], 10)
+    assert (kout[0], status[0], alpha[0, 0]) == (1, IMPED_ERR_BREAKDOWN, 3.0)
+    assert (kout[1], status[1]) == (10, 0)
+    assert (kout[2], status[2]) == (0, 0)
