@@ -1,16 +1,16 @@
 // Surrogate network kernels: an ensemble of E fully connected GELU networks
 // of identical shape, trained and evaluated together (blockIdx.z = member).
 //
-// * gemm_bf16_kernel: C[m][n] = sum_k A(m,k) B(n,k) on the matrix cores
-//   (v_mfma_f32_32x32x8 bf16, FP32 accumulation), 64x64 output tiles of four
-//   waves, 32-deep K slices staged through LDS; either operand may be stored
-//   k-contiguous or row-contiguous, so forward (X W^T), input gradient
-//   (dZ W) and weight gradient (dZ^T X) are one kernel.  Epilogues fuse the
-//   bias, GELU (pre-activation kept in FP32 for the backward pass) and the
-//   GELU derivative.
-// * mse_grad_kernel, bias_grad_kernel, adam_kernel, gather_kernel: loss
-//   gradient, bias gradients, the Adam update (FP32 master weights, BF16
-//   copies for the GEMMs) and minibatch assembly.
+// * gemm_nt_kernel: every GEMM, C[m][n] = sum_k A[m][k] B[n][k] with both
+//   operands k-contiguous and padded to whole tiles: forward (X W^T), input gradient (dZ W, from a transposed copy of W) and weight
+//   gradient (dZ^T X, from transposed copies that the producing epilogues
+//   write).  Epilogues fuse the bias, GELU (pre-activation kept in FP32 for the
+//   backward pass), the loss and its gradient, the GELU derivative, the bias
+//   gradients and the Adam update.
+// * gather_kernel, loss_sum_kernel: minibatch inputs and the losses.
+//
+// BF16 copies of weights and activations are stored with rows padded to a
+// multiple of 64 entries, the padding zero, so no load is bounds-checked.
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -63,136 +63,36 @@ __device__ __forceinline__ float gelu_inference(float x) {
   return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f));
 }
 
-enum { EPI_BIAS_GELU = 0, EPI_BIAS = 1, EPI_DGELU = 2, EPI_F32 = 3 };
+constexpr int TM = 64, TN = 64;
 
-struct GemmArgs {
-  const uint16_t* A;  // AK: A(m,k) = A[m*lda + k]; else A[k*lda + m]
+enum { NT_GELU, NT_MSE, NT_DGELU, NT_GRAD, NT_ADAM, NT_HIDDEN, NT_OUT };
+
+// gemm_nt_kernel: M, N rows of A and B that hold data, out of mp, np (multiples
+// of 64; rows between are zero or meet zeros), K a multiple of 64.
+struct NtArgs {
+  const uint16_t* A;
   int64_t lda, a_z;
-  const uint16_t* B;  // BK: B(n,k) = B[n*ldb + k]; else B[k*ldb + n]
+  const uint16_t* B;
   int64_t ldb, b_z;
-  int M, N, K;
-  float* Cf;  // row-major [M][ldc]
-  uint16_t* Cb;
-  int64_t ldc, c_z;
-  const float* bias;  // [N] per member
+  int M, N, mp, np, K;
+  const float* bias;  // forward: [N] per member
   int64_t bias_z;
-  const float* aux;  // EPI_DGELU: pre-activation, layout of C
-  int vec;           // gemm_fwd_kernel: K, lda, ldb, a_z, b_z multiples of 8, A and B 16-byte aligned
-  const float* Af;   // gemm_fwd_kernel<EPI, true>: A in FP32 (shared by the members), rounded to BF16 when staged
+  const float* Af;  // with AF: A in FP32 [M][lda] (shared by the members), entries past lda taken as 0
+  float* out;       // NT_OUT: result [M][N] per member
+  float* z;      // NT_GELU: pre-activations written, NT_DGELU: read; [mp][np]
+  uint16_t* C;   // NT_GELU, NT_MSE, NT_DGELU, NT_HIDDEN: BF16 result [mp][np]
+  uint16_t* CT;  //   (but NT_HIDDEN) and transposed [np][mp]; both per member mp * np
+  // NT_MSE: targets (row idx[m], or m without idx) and the sum of squares of each tile
+  const float* T;
+  const int32_t* idx;
+  double* lossp;
+  // NT_GRAD, NT_ADAM: gradient or parameters of the layer, flat [M][N], then the biases [M]
+  float *g, *w, *m, *v;
+  int64_t p_z, b_off;
+  uint16_t *wb, *wbT;  // NT_ADAM: BF16 copies [mp][np] and [np][mp]
+  int64_t wb_z;
+  float lr, b1, b2, eps, bc1, bc2;
 };
-
-constexpr int TM = 64, TN = 64, TK = 32, LK = TK + 8;
-
-// Stage a 64 x 32 slice (rows r0.., k0..) of an operand into tile[row][k],
-// zero outside [0, R) x [0, K).
-template <bool KC>
-__device__ __forceinline__ void stage(const uint16_t* src, int64_t ld, int R, int K, int r0, int k0,
-                                      uint16_t (*tile)[LK], int t) {
-  if constexpr (KC) {
-    const int r = t >> 2, kc = (t & 3) * 8;
-    const int gr = r0 + r, gk = k0 + kc;
-    uint16_t v[8];
-    const uint16_t* p = src + (int64_t)gr * ld + gk;
-    if (gr < R && gk + 8 <= K && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
-      *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(p);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (gr < R && gk + i < K) ? src[(int64_t)gr * ld + gk + i] : (uint16_t)0;
-    }
-    *reinterpret_cast<uint4*>(&tile[r][kc]) = *reinterpret_cast<const uint4*>(v);
-  } else {
-    const int k = t >> 3, rc = (t & 7) * 8;
-    const int gk = k0 + k, gr = r0 + rc;
-    uint16_t v[8];
-    const uint16_t* p = src + (int64_t)gk * ld + gr;
-    if (gk < K && gr + 8 <= R && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
-      *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(p);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = (gk < K && gr + i < R) ? src[(int64_t)gk * ld + gr + i] : (uint16_t)0;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) tile[rc + i][k] = v[i];
-  }
-}
-
-template <bool AK, bool BK, int EPI>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
-  __shared__ __align__(16) uint16_t As[TM][LK];
-  __shared__ __align__(16) uint16_t Bs[TN][LK];
-  const int z = blockIdx.z;
-  const uint16_t* A = g.A + (int64_t)z * g.a_z;
-  const uint16_t* B = g.B + (int64_t)z * g.b_z;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  f32x16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  for (int k0 = 0; k0 < g.K; k0 += TK) {
-    stage<AK>(A, g.lda, g.M, g.K, m0, k0, As, t);
-    stage<BK>(B, g.ldb, g.N, g.K, n0, k0, Bs, t);
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < TK; kk += 16) {
-      // 16-deep steps (gfx950): lane l supplies row l%32 and k = kk + 8*(l/32) .. +7
-      // of each operand (rows of LK = 40 elements keep every read 16-byte aligned)
-      const int kq = kk + 8 * (lane >> 5);
-      const uint4 a = *reinterpret_cast<const uint4*>(&As[wm + (lane & 31)][kq]);
-      const uint4 b = *reinterpret_cast<const uint4*>(&Bs[wn + (lane & 31)][kq]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc,
-                                                    0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
-  // (the column's bias read once and added before the first store)
-  const int64_t cz = (int64_t)z * g.c_z;
-  const int n = n0 + wn + (lane & 31);
-  constexpr bool with_bias = EPI == EPI_BIAS_GELU || EPI == EPI_BIAS;
-  const float bn = with_bias && n < g.N ? g.bias[(int64_t)z * g.bias_z + n] : 0.0f;
-  float zr[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    zr[r] = with_bias ? acc[r] + bn : acc[r];
-    asm volatile("" : "+v"(zr[r]));  // no instruction: keeps the sum here, out of the branches below
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    if (m >= g.M || n >= g.N) continue;
-    const int64_t o = cz + (int64_t)m * g.ldc + n;
-    const float v = zr[r];
-    if constexpr (EPI == EPI_BIAS_GELU) {
-      g.Cf[o] = v;
-      g.Cb[o] = f2bf(gelu(v));
-    } else if constexpr (EPI == EPI_BIAS) {
-      g.Cf[o] = v;
-    } else if constexpr (EPI == EPI_DGELU) {
-      g.Cb[o] = f2bf(v * gelu_grad(g.aux[o]));
-    } else {
-      g.Cf[o] = v;
-    }
-  }
-}
-
-// Forward GEMM C = X W^T (+ bias, GELU) with K staged FK at a time for both
-// 64-row operand tiles: every global load of a stage is in flight together
-// and one barrier precedes its MFMAs, so a 512-deep layer pays two load
-// latencies instead of sixteen.  2 x 64 x (FK + 8) bf16 = 66 KiB of LDS, so
-// two workgroups share a CU (the 1000-wide output layer has 320 of them).
-constexpr int FK = 256, FLK = FK + 8;
-constexpr size_t FWD_LDS = (size_t)2 * TM * FLK * sizeof(uint16_t);
-
-// 8 consecutive bf16 of row gr from column gk (zeros outside [0, R) x [0, K)).
-__device__ __forceinline__ uint4 load8(const uint16_t* src, int64_t ld, int R, int K, int gr, int gk) {
-  const uint16_t* p = src + (int64_t)gr * ld + gk;
-  if (gr < R && gk + 8 <= K && (reinterpret_cast<uintptr_t>(p) & 15) == 0) return *reinterpret_cast<const uint4*>(p);
-  uint16_t v[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = (gr < R && gk + i < K) ? src[(int64_t)gr * ld + gk + i] : (uint16_t)0;
-  return *reinterpret_cast<const uint4*>(v);
-}
 
 // Eight FP32 values rounded to BF16, packed as the BF16 row chunk.
 __device__ __forceinline__ uint4 pack_bf16x8(const float4& a, const float4& b) {
@@ -204,162 +104,245 @@ __device__ __forceinline__ uint4 pack_bf16x8(const float4& a, const float4& b) {
   return r;
 }
 
-// AF: the A operand is FP32 (g.Af, vec path only; the predictions' first
-// layer reads the batch inputs straight from mapped host memory, so no
-// conversion launch precedes it).
-template <int EPI, bool AF>
-__global__ __launch_bounds__(256) void gemm_fwd_kernel(GemmArgs g) {
-  extern __shared__ __align__(16) uint16_t fsm[];
-  uint16_t(*As)[FLK] = reinterpret_cast<uint16_t(*)[FLK]>(fsm);
-  uint16_t(*Bs)[FLK] = reinterpret_cast<uint16_t(*)[FLK]>(fsm + TM * FLK);
-  // Tile order for the eight XCDs, which take the workgroups round-robin in
-  // launch order (x fastest) and each have their own L2: with the launch
-  // order, XCD i got output-column tile i of every row tile and member, so
-  // each XCD fetched every activation tile (eight fetches per tile).
-  // Renumbered so that each XCD takes one contiguous run of tiles, ordered
-  // member, column tile, row tile (rows fastest): an XCD's run covers whole
-  // columns of one or two members, every weight tile is fetched by one XCD
-  // and every activation tile by about two.  Same arithmetic per tile.
-  int z = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
-  {
-    const int gx = gridDim.x, gy = gridDim.y, tiles = gx * gy * gridDim.z;
-    if ((tiles & 7) == 0) {
-      const int l = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
-      const int q = (l & 7) * (tiles >> 3) + (l >> 3);  // a bijection of [0, tiles) when 8 | tiles
-      z = q / (gx * gy);
-      const int r = q - z * gx * gy;
-      bx = r / gy;
-      by = r - bx * gy;
-    }
+// Adam step of one parameter from its gradient; returns the new value.
+__device__ __forceinline__ float adam_step(const NtArgs& a, int64_t o, float g) {
+  const float mi = a.b1 * a.m[o] + (1.0f - a.b1) * g;
+  const float vi = a.b2 * a.v[o] + (1.0f - a.b2) * g * g;
+  a.m[o] = mi;
+  a.v[o] = vi;
+  const float w = a.w[o] - a.lr * (mi / a.bc1) / (sqrtf(vi / a.bc2) + a.eps);
+  a.w[o] = w;
+  return w;
+}
+
+// blockIdx -> (member, column tile, row tile) for the eight XCDs, which take the
+// workgroups round-robin in launch order (x fastest) and each have their own L2:
+// with the launch order, XCD i got output-column tile i of every row tile and
+// member, so each XCD fetched every activation tile (eight fetches per tile).
+// Renumbered so that each XCD takes one contiguous run of tiles, ordered
+// member, column tile, row tile (rows fastest): an XCD's run covers whole
+// columns of one or two members, every weight tile is fetched by one XCD and
+// every activation tile by about two.  Same arithmetic per tile.
+__device__ __forceinline__ void xcd_tile(int& z, int& bx, int& by) {
+  z = blockIdx.z, bx = blockIdx.x, by = blockIdx.y;
+  const int gx = gridDim.x, gy = gridDim.y, tiles = gx * gy * gridDim.z;
+  if ((tiles & 7) == 0) {
+    const int l = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const int q = (l & 7) * (tiles >> 3) + (l >> 3);  // a bijection of [0, tiles) when 8 | tiles
+    z = q / (gx * gy);
+    const int r = q - z * gx * gy;
+    bx = r / gy;
+    by = r - bx * gy;
   }
-  const uint16_t* A = AF ? nullptr : g.A + (int64_t)z * g.a_z;
-  const uint16_t* B = g.B + (int64_t)z * g.b_z;
+}
+
+// One 64 x 64 tile per workgroup of four waves (a 32 x 32 accumulator each), K
+// in steps of 64 through two LDS buffers: the next step's 16-byte loads are in
+// flight while this step's four MFMAs per wave run, one barrier a step.
+//
+// What bounds it: at these sizes a launch is a few dependent load latencies
+// plus the epilogue's stores; small tiles, because 1024 x 512 outputs of five
+// members are only 640 of them.  Measured, five members of 8-512-512-512-1000
+// on one MI355X: a 512 x 512 layer at 256 rows 9.9 -> 8.3 us a launch, at 1001
+// rows 18.6 -> 11.2 us (both against K staged 256 deep, bounds-checked); a
+// training step of 1024 rows 1.63 -> 0.24 ms, of which the separate bias
+// gradients (one thread per column, 220 us a layer), the loss (an FP64 atomic
+// per 256 values, 242 us) and transposing loads were 1.3 ms.
+template <int EPI, bool AF = false>
+__global__ __launch_bounds__(256) void gemm_nt_kernel(NtArgs g) {
+  constexpr int SK = 64, LK = SK + 8;  // rows of 144 bytes spread over the banks
+  __shared__ __align__(16) uint16_t As[2][TM][LK], Bs[2][TN][LK];
+  __shared__ double red[4];
+  int z, bx, by;
+  xcd_tile(z, bx, by);
   const int m0 = by * TM, n0 = bx * TN;
   const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int sr = t >> 2, sc = (t & 3) * 16;  // this thread's staged row and its 16 entries
+  const uint16_t* pa = AF ? nullptr : g.A + (int64_t)z * g.a_z + (int64_t)(m0 + sr) * g.lda + sc;
+  // AF: rows past M read the last one (their outputs are dropped)
+  const float* paf = AF ? g.Af + (int64_t)(m0 + sr < g.M ? m0 + sr : g.M - 1) * g.lda + sc : nullptr;
+  const auto load_a = [&](int k, uint4& lo, uint4& hi) {
+    if constexpr (AF) {
+      lo = hi = make_uint4(0, 0, 0, 0);
+      if (sc + k < g.lda)
+        lo = pack_bf16x8(*reinterpret_cast<const float4*>(paf + k), *reinterpret_cast<const float4*>(paf + k + 4));
+      if (sc + k + 8 < g.lda)
+        hi = pack_bf16x8(*reinterpret_cast<const float4*>(paf + k + 8), *reinterpret_cast<const float4*>(paf + k + 12));
+    } else {
+      lo = *reinterpret_cast<const uint4*>(pa + k);
+      hi = *reinterpret_cast<const uint4*>(pa + k + 8);
+    }
+  };
+  const uint16_t* pb = g.B + (int64_t)z * g.b_z + (int64_t)(n0 + sr) * g.ldb + sc;
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-  for (int k0 = 0; k0 < g.K; k0 += FK) {
-    const int kc8 = ((g.K - k0 < FK ? g.K - k0 : FK) + 7) & ~7;  // MFMA steps of 8, zero padded
-    const int per_row = kc8 / 8;
-    const int chunks = TM * per_row;
-    if (g.vec) {
-      // every load of the stage issued before the first LDS write; rows past
-      // M or N read the last row instead (their outputs are not stored), so
-      // no load waits behind a branch
-      // (chunk indices past the stage repeat its last chunk: those threads
-      // write the same values to the same LDS slot, so nothing branches)
-      uint4 ra[8], rb[8];
-      float4 fa[AF ? 8 : 1][2];
-      int slot[8];
+  constexpr bool weights = EPI == NT_GRAD || EPI == NT_ADAM;
+  const bool row_sums = weights && bx == 0;  // the bias gradients: sums of A's rows
+  float rs = 0.0f;
+  uint4 a0, a1;
+  load_a(0, a0, a1);
+  uint4 b0 = *reinterpret_cast<const uint4*>(pb), b1 = *reinterpret_cast<const uint4*>(pb + 8);
+  for (int k0 = 0, buf = 0; k0 < g.K; k0 += SK, buf ^= 1) {
+    *reinterpret_cast<uint4*>(&As[buf][sr][sc]) = a0;
+    *reinterpret_cast<uint4*>(&As[buf][sr][sc + 8]) = a1;
+    *reinterpret_cast<uint4*>(&Bs[buf][sr][sc]) = b0;
+    *reinterpret_cast<uint4*>(&Bs[buf][sr][sc + 8]) = b1;
+    if (row_sums) {
+      const uint32_t u[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int c = t + 256 * i < chunks ? t + 256 * i : chunks - 1;
-        const int r = c / per_row, k8 = (c - r * per_row) * 8;
-        slot[i] = r * FLK + k8;
-        const int ga = m0 + r < g.M ? m0 + r : g.M - 1, gb = n0 + r < g.N ? n0 + r : g.N - 1;
-        if constexpr (AF) {
-          const float* pa = g.Af + (int64_t)ga * g.lda + k0 + k8;
-          fa[i][0] = *reinterpret_cast<const float4*>(pa);
-          fa[i][1] = *reinterpret_cast<const float4*>(pa + 4);
-        } else {
-          ra[i] = *reinterpret_cast<const uint4*>(A + (int64_t)ga * g.lda + k0 + k8);
-        }
-        rb[i] = *reinterpret_cast<const uint4*>(B + (int64_t)gb * g.ldb + k0 + k8);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if constexpr (AF) ra[i] = pack_bf16x8(fa[i][0], fa[i][1]);
-        *reinterpret_cast<uint4*>(&As[0][0] + slot[i]) = ra[i];
-        *reinterpret_cast<uint4*>(&Bs[0][0] + slot[i]) = rb[i];
-      }
-    } else if constexpr (!AF) {
-#pragma unroll 8
-      for (int c = t; c < chunks; c += 256) {
-        const int r = c / per_row, k8 = (c - r * per_row) * 8;
-        const uint4 va = load8(A, g.lda, g.M, g.K, m0 + r, k0 + k8);
-        const uint4 vb = load8(B, g.ldb, g.N, g.K, n0 + r, k0 + k8);
-        *reinterpret_cast<uint4*>(&As[r][k8]) = va;
-        *reinterpret_cast<uint4*>(&Bs[r][k8]) = vb;
-      }
+      for (int i = 0; i < 8; ++i) rs += __uint_as_float(u[i] << 16) + __uint_as_float(u[i] & 0xffff0000u);
     }
     __syncthreads();
-    int kk = 0;
-    for (; kk + 16 <= kc8; kk += 16) {
-      // 16-deep steps (gfx950): lane l supplies row l%32 and k = kk + 8*(l/32) .. +7
-      // of each operand; both operands use the same k assignment
+    if (k0 + SK < g.K) {
+      load_a(k0 + SK, a0, a1);
+      b0 = *reinterpret_cast<const uint4*>(pb + k0 + SK);
+      b1 = *reinterpret_cast<const uint4*>(pb + k0 + SK + 8);
+    }
+#pragma unroll
+    for (int kk = 0; kk < SK; kk += 16) {
+      // lane l supplies row l%32 and k = kk + 8*(l/32) .. +7 of each operand
       const int kq = kk + 8 * (lane >> 5);
-      const uint4 a = *reinterpret_cast<const uint4*>(&As[wm + (lane & 31)][kq]);
-      const uint4 b = *reinterpret_cast<const uint4*>(&Bs[wn + (lane & 31)][kq]);
+      const uint4 a = *reinterpret_cast<const uint4*>(&As[buf][wm + (lane & 31)][kq]);
+      const uint4 b = *reinterpret_cast<const uint4*>(&Bs[buf][wn + (lane & 31)][kq]);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc,
                                                     0, 0, 0);
     }
-    if (kk < kc8) {
-      // an odd 8-deep step: lane l supplies row l%32 and k = kk + 4*(l/32) .. +3
-      const int kq = kk + 4 * (lane >> 5);
-      const bf16x4 a = *reinterpret_cast<const bf16x4*>(&As[wm + (lane & 31)][kq]);
-      const bf16x4 b = *reinterpret_cast<const bf16x4*>(&Bs[wn + (lane & 31)][kq]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
+  }
+  // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32
+  const int n = n0 + wn + (lane & 31), mb = m0 + wm + 4 * (lane >> 5);
+  if constexpr (weights) {
+    if (row_sums) {  // the four threads of a row
+      rs += __shfl_xor(rs, 1);
+      rs += __shfl_xor(rs, 2);
+      if ((t & 3) == 0 && m0 + sr < g.M) {
+        const int64_t o = (int64_t)z * g.p_z + g.b_off + m0 + sr;
+        if constexpr (EPI == NT_GRAD)
+          g.g[o] = rs;
+        else
+          adam_step(g, o, rs);
+      }
     }
-    __syncthreads();
-  }
-  // accumulator r of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32.
-  // The column's bias is read once and added to every accumulator before the
-  // first store: read after each store (as a pointer that may alias the
-  // output would be), or first used inside the per-row branches, it puts a
-  // wait for every earlier store (stores count in vmcnt) between the stores.
-  const int64_t cz = (int64_t)z * g.c_z;
-  const int n = n0 + wn + (lane & 31);
-  const float bn = n < g.N ? g.bias[(int64_t)z * g.bias_z + n] : 0.0f;
-  float zr[16];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    zr[r] = acc[r] + bn;
-    asm volatile("" : "+v"(zr[r]));  // no instruction: keeps the sum here, out of the branches below
-  }
+    for (int q = 0; q < 4; ++q) {
+      uint16_t h[4];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int m = m0 + wm + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-    if (m >= g.M || n >= g.N) continue;
-    const int64_t o = cz + (int64_t)m * g.ldc + n;
-    const float zv = zr[r];
-    if (EPI != EPI_BIAS_GELU || g.Cf) g.Cf[o] = zv;  // hidden layers of a prediction keep no pre-activation
-    if constexpr (EPI == EPI_BIAS_GELU) g.Cb[o] = f2bf(g.Cf ? gelu(zv) : gelu_inference(zv));
+      for (int r = 0; r < 4; ++r) {
+        const int m = mb + 8 * q + r;
+        const int64_t o = (int64_t)z * g.p_z + (int64_t)m * g.N + n;
+        h[r] = 0;
+        if (m < g.M && n < g.N) {
+          if constexpr (EPI == NT_GRAD) {
+            g.g[o] = acc[4 * q + r];
+          } else {
+            h[r] = f2bf(adam_step(g, o, acc[4 * q + r]));
+            g.wb[(int64_t)z * g.wb_z + (int64_t)m * g.np + n] = h[r];
+          }
+        }
+      }
+      if constexpr (EPI == NT_ADAM)
+        *reinterpret_cast<uint2*>(g.wbT + (int64_t)z * g.wb_z + (int64_t)n * g.mp + mb + 8 * q) =
+            make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+    }
+  } else if constexpr (EPI == NT_OUT || EPI == NT_HIDDEN) {
+    // the column's bias read once and added to every accumulator before the
+    // first store: first used inside the per-row branches, it would put a wait
+    // for every earlier store between the stores
+    const float bn = n < g.N ? g.bias[(int64_t)z * g.bias_z + n] : 0.0f;
+    float v[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      v[r] = acc[r] + bn;
+      asm volatile("" : "+v"(v[r]));  // no instruction: keeps the sum here
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int m = mb + 8 * (r >> 2) + (r & 3);
+      if constexpr (EPI == NT_HIDDEN)
+        g.C[((int64_t)z * g.mp + m) * g.np + n] = f2bf(gelu_inference(v[r]));
+      else if (m < g.M && n < g.N)
+        g.out[((int64_t)z * g.M + m) * g.N + n] = v[r];
+    }
+  } else {
+    const int64_t cz = (int64_t)z * g.mp * g.np;
+    float bn = 0.0f;
+    if constexpr (EPI != NT_DGELU) bn = n < g.N ? g.bias[(int64_t)z * g.bias_z + n] : 0.0f;
+    double sq = 0.0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint16_t h[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = mb + 8 * q + r;
+        const int64_t o = cz + (int64_t)m * g.np + n;
+        const float v = acc[4 * q + r] + bn;
+        if constexpr (EPI == NT_GELU) {
+          g.z[o] = v;
+          h[r] = f2bf(gelu(v));
+        } else if constexpr (EPI == NT_DGELU) {
+          h[r] = f2bf(v * gelu_grad(g.z[o]));
+        } else {
+          h[r] = 0;
+          if (m < g.M && n < g.N) {
+            const float d = v - g.T[(int64_t)(g.idx ? g.idx[m] : m) * g.N + n];
+            h[r] = f2bf(2.0f * d / (float)((int64_t)g.M * g.N));
+            sq += (double)d * (double)d;
+          }
+        }
+        g.C[o] = h[r];
+      }
+      *reinterpret_cast<uint2*>(g.CT + cz + (int64_t)n * g.mp + mb + 8 * q) =
+          make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+    }
+    if constexpr (EPI == NT_MSE) {
+      sq = wave_sum(sq);
+      if (lane == 0) red[wave] = sq;
+      __syncthreads();
+      if (t == 0) g.lossp[((int64_t)z * gridDim.y + by) * gridDim.x + bx] = red[0] + red[1] + red[2] + red[3];
+    }
   }
 }
 
-__global__ void to_bf16_kernel(const float* x, int64_t n, uint16_t* y) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) y[i] = f2bf(x[i]);
-}
-
-// minibatch rows idx[b] of the data set: inputs to BF16, targets as FP32
-__global__ void gather_kernel(const float* X, int dx, const float* Y, int dy, const int32_t* idx, int B,
-                              uint16_t* xb, float* yb) {
-  const int b = blockIdx.x;
-  if (b >= B) return;
-  const int64_t r = idx[b];
-  for (int j = threadIdx.x; j < dx; j += blockDim.x) xb[(int64_t)b * dx + j] = f2bf(X[r * dx + j]);
-  for (int j = threadIdx.x; j < dy; j += blockDim.x) yb[(int64_t)b * dy + j] = Y[r * dy + j];
-}
-
-// dY = 2 (Y - T) / (B N) in BF16 per member; loss[z] += sum (Y - T)^2 / (B N)
-__global__ __launch_bounds__(256) void mse_grad_kernel(const float* Y, const float* T, int64_t BN, uint16_t* dY,
-                                                       double* loss) {
-  __shared__ double red[4];
-  const int z = blockIdx.y;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+// out[i] = sum of part[i*tiles ..] / count, one wave per value
+__global__ __launch_bounds__(64) void loss_sum_kernel(const double* part, int tiles, double count, double* out) {
   double s = 0.0;
-  if (i < BN) {
-    const float d = Y[(int64_t)z * BN + i] - T[i];
-    dY[(int64_t)z * BN + i] = f2bf(2.0f * d / (float)BN);
-    s = (double)d * (double)d;
+  for (int k = threadIdx.x; k < tiles; k += 64) s += part[(int64_t)blockIdx.x * tiles + k];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) out[blockIdx.x] = s / count;
+}
+
+// x [B][d] in BF16 with rows padded to ld entries (the padding stays zero)
+__global__ void to_bf16_kernel(const float* x, int64_t n, int d, int ld, uint16_t* y) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i / d * ld + i % d] = f2bf(x[i]);
+}
+
+// BF16 copies of one layer's weights W [out][in] of every member: wb [op][ip]
+// and its transpose wbT [ip][op], zero-padded (members w_z and wb_z apart)
+__global__ void pack_weights_kernel(const float* w, int64_t w_z, int out, int in, int op, int ip, uint16_t* wb,
+                                    uint16_t* wbT, int64_t wb_z) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= (int64_t)op * ip) return;
+  const int64_t z = blockIdx.y;
+  const int o = (int)(i / ip), k = (int)(i % ip);
+  wb[z * wb_z + i] = o < out && k < in ? f2bf(w[z * w_z + (int64_t)o * in + k]) : (uint16_t)0;
+  const int kt = (int)(i / op), ot = (int)(i % op);
+  wbT[z * wb_z + i] = ot < out && kt < in ? f2bf(w[z * w_z + (int64_t)ot * in + kt]) : (uint16_t)0;
+}
+
+// minibatch inputs (row idx[b] of X, or b without idx) in BF16, xb [bp][ld]
+// and xT [ld][bp]; rows from B on are zero
+__global__ void gather_kernel(const float* X, int dx, const int32_t* idx, int B, int bp, int ld, uint16_t* xb,
+                              uint16_t* xT) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= bp) return;
+  const int64_t r = b < B ? (idx ? idx[b] : b) : 0;
+  for (int j = 0; j < dx; ++j) {
+    const uint16_t h = b < B ? f2bf(X[r * dx + j]) : (uint16_t)0;
+    xb[(int64_t)b * ld + j] = h;
+    xT[(int64_t)j * bp + b] = h;
   }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(&loss[z], (red[0] + red[1] + red[2] + red[3]) / (double)BN);
 }
 
 // Sum over a 256-thread workgroup, broadcast to every thread.
@@ -511,65 +494,13 @@ __global__ __launch_bounds__(256) void ensemble_stats_reg_kernel(const float* y,
   }
 }
 
-// db[z][n] = sum_b dZ[z][b][n]
-__global__ void bias_grad_kernel(const uint16_t* dZ, int B, int N, int64_t dz_z, float* db, int64_t db_z) {
-  const int z = blockIdx.y;
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.0f;
-  for (int b = 0; b < B; ++b) s += bf2f(dZ[(int64_t)z * dz_z + (int64_t)b * N + n]);
-  db[(int64_t)z * db_z + n] = s;
-}
-
-__global__ void adam_kernel(float* w, const float* g, float* m, float* v, uint16_t* wb, int64_t n, float lr, float b1,
-                            float b2, float eps, float bc1, float bc2) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float wi = w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-  w[i] = wi;
-  wb[i] = f2bf(wi);
-}
-
-template <bool AK, bool BK, int EPI>
-void gemm(const GemmArgs& g, int E, hipStream_t s) {
-  const dim3 grid(blocks_for(g.N, TN), blocks_for(g.M, TM), E);
-  hipLaunchKernelGGL((gemm_bf16_kernel<AK, BK, EPI>), grid, dim3(256), 0, s, g);
-  HIP_CHECK(hipGetLastError());
-}
-
-// forward layer (X W^T + bias, GELU or not) by the whole-K kernel
 template <int EPI, bool AF = false>
-void fwd_attr() {
-  static bool attr = false;
-  if (!attr) {
-    HIP_CHECK(hipFuncSetAttribute((const void*)gemm_fwd_kernel<EPI, AF>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)FWD_LDS));
-    attr = true;
-  }
-}
-
-template <int EPI>
-void gemm_fwd(const GemmArgs& g0, int E, hipStream_t s) {
-  GemmArgs g = g0;
-  const void* a = g.Af ? (const void*)g.Af : (const void*)g.A;
-  g.vec = g.K % 8 == 0 && g.lda % 8 == 0 && g.ldb % 8 == 0 && g.a_z % 8 == 0 && g.b_z % 8 == 0 &&
-          (reinterpret_cast<uintptr_t>(a) & 15) == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
-  const dim3 grid(blocks_for(g.N, TN), blocks_for(g.M, TM), E);
-  if (g.Af) {
-    if (!g.vec) throw std::runtime_error("gemm_fwd: an FP32 operand needs K, strides and alignment in steps of 8");
-    fwd_attr<EPI, true>();
-    hipLaunchKernelGGL((gemm_fwd_kernel<EPI, true>), grid, dim3(256), FWD_LDS, s, g);
-  } else {
-    fwd_attr<EPI>();
-    hipLaunchKernelGGL((gemm_fwd_kernel<EPI, false>), grid, dim3(256), FWD_LDS, s, g);
-  }
+void gemm_nt(const NtArgs& g, int E, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_nt_kernel<EPI, AF>), dim3(g.np / TN, g.mp / TM, E), dim3(256), 0, s, g);
   HIP_CHECK(hipGetLastError());
 }
+
+inline int pad64(int n) { return (n + 63) / 64 * 64; }
 
 }  // namespace
 
@@ -607,11 +538,17 @@ struct Mlp {
   std::vector<int64_t> w_off, b_off;  // per layer offsets in a member's flat parameter vector
   int64_t P = 0;                    // parameters per member
   int64_t step = 0;                 // Adam steps taken
-  DevBuf w, wb, g, m, v;            // [E][P] fp32 master, bf16 copy, gradient, Adam moments
+  std::vector<int> pd;              // widths padded to multiples of 64
+  std::vector<int64_t> wbo;         // per layer offsets in a member's BF16 weights
+  int64_t PB = 0;                   // BF16 weights per member
+  DevBuf w, g, m, v;                // [E][P] fp32 master, gradient, Adam moments
+  DevBuf wb, wbT;                   // [E][PB] bf16 weights: layer l [pd[l+1]][pd[l]], and transposed
   static constexpr int MAXL = 16;
-  DevBuf zf[MAXL], hb[MAXL], dz[MAXL];  // per layer: pre-activation fp32, activation bf16, dZ bf16
-  bool acts = false;
-  DevBuf xb, yb, out, loss, idx;    // minibatch input bf16, targets fp32, output fp32 [E][B][dL]
+  // per layer: activation bf16 [E][rows][pd[l+1]] (rows: the batch padded to a
+  // multiple of 64); training: transposed, pre-activation fp32, dZ and transposed
+  DevBuf hb[MAXL], hT[MAXL], zf[MAXL], dz[MAXL], dzT[MAXL];
+  int act_rows = 0, train_rows = 0;
+  DevBuf xb, xT, out, loss;         // minibatch input bf16 [rows][pd[0]], transposed; output fp32 [E][B][dL]; losses
   DevBuf dX, dY;                    // data set (fp32)
   DevBuf sw, smean, st;             // ensemble statistics: area weights, mean [B][dL], misfit target [dL]
   HostIO xin, sout;                 // batch input x [B][d0] (fp32); disagreement [B] and misfit [B]
@@ -634,116 +571,180 @@ struct Mlp {
 
 namespace {
 
-void alloc_acts(Mlp& net, int B) {
-  if (B <= net.max_batch && net.acts) return;
-  net.max_batch = std::max(B, net.max_batch);
-  net.acts = true;
-  const int64_t Bm = net.max_batch;
-  for (int l = 0; l < net.L; ++l) {
-    const int64_t out = net.dims[l + 1];
-    net.zf[l].reserve(net.E * Bm * out * 4);
-    net.hb[l].reserve(net.E * Bm * out * 2);
-    net.dz[l].reserve(net.E * Bm * out * 2);
-  }
-  net.xb.reserve(Bm * net.dims[0] * 2);
-  net.yb.reserve(Bm * net.dims[net.L] * 4);
-  net.out.reserve(net.E * Bm * net.dims[net.L] * 4);
-  net.idx.reserve(Bm * 4);
-  net.loss.reserve(net.E * 8);
+// A buffer of n bytes, all zero when it had to grow (the padding of BF16
+// arrays is written by nobody, so it stays zero whatever the batch).
+void reserve_zero(DevBuf& b, size_t n, hipStream_t s) {
+  if (n <= b.bytes) return;
+  b.reserve(n);
+  HIP_CHECK(hipMemsetAsync(b.p, 0, b.bytes, s));
 }
 
-// forward pass of every member on the BF16 minibatch in xb; output in out
-// x_f32: the first layer reads FP32 inputs there (else the BF16 copy in xb);
-// inference: the hidden layers' FP32 pre-activations (kept for the backward
-// pass) are not written
-void forward(Mlp& net, int B, hipStream_t s, const float* x_f32 = nullptr, bool inference = false) {
-  const uint16_t* x = net.xb.as<uint16_t>();
-  int64_t x_z = 0;  // the input is shared by all members
+void alloc_acts(Mlp& net, int B, hipStream_t s) {
+  const int rows = pad64(std::max(B, net.max_batch));
+  if (rows <= net.act_rows) return;
+  for (int l = 0; l + 1 < net.L; ++l) reserve_zero(net.hb[l], (size_t)net.E * rows * net.pd[l + 1] * 2, s);
+  reserve_zero(net.xb, (size_t)rows * net.pd[0] * 2, s);
+  net.out.reserve((size_t)net.E * rows * net.dims[net.L] * 4);
+  net.act_rows = rows;
+}
+
+void alloc_train(Mlp& net, int B, hipStream_t s) {
+  alloc_acts(net, B, s);
+  const int rows = net.act_rows;
+  if (rows <= net.train_rows) return;
   for (int l = 0; l < net.L; ++l) {
-    const int in = net.dims[l], outd = net.dims[l + 1];
-    GemmArgs g{};
-    g.A = x;
-    if (l == 0) g.Af = x_f32;
-    g.lda = in;
-    g.a_z = x_z;
-    g.B = net.wb.as<uint16_t>() + net.w_off[l];
-    g.ldb = in;
-    g.b_z = net.P;
+    const size_t n = (size_t)net.E * rows * net.pd[l + 1];
+    if (l + 1 < net.L) {
+      reserve_zero(net.hT[l], n * 2, s);
+      net.zf[l].reserve(n * 4);
+    }
+    net.dz[l].reserve(n * 2);
+    net.dzT[l].reserve(n * 2);
+  }
+  reserve_zero(net.xT, (size_t)rows * net.pd[0] * 2, s);
+  net.train_rows = rows;
+}
+
+// Forward pass of a prediction: every member on B samples, outputs in out.
+// x_f32: the first layer reads FP32 inputs there (else the BF16 copy in xb).
+void forward(Mlp& net, int B, hipStream_t s, const float* x_f32 = nullptr) {
+  const int rows = pad64(B);
+  for (int l = 0; l < net.L; ++l) {
+    NtArgs g{};
+    g.A = l ? net.hb[l - 1].as<uint16_t>() : net.xb.as<uint16_t>();
+    g.lda = g.K = net.pd[l];
+    g.a_z = l ? (int64_t)rows * net.pd[l] : 0;
+    g.B = net.wb.as<uint16_t>() + net.wbo[l];
+    g.ldb = net.pd[l];
+    g.b_z = net.PB;
     g.M = B;
-    g.N = outd;
-    g.K = in;
-    g.ldc = outd;
-    g.c_z = (int64_t)B * outd;
+    g.N = net.dims[l + 1];
+    g.mp = rows;
+    g.np = net.pd[l + 1];
+    g.bias = net.w.as<float>() + net.b_off[l];
+    g.bias_z = net.P;
+    g.C = net.hb[l].as<uint16_t>();
+    g.out = net.out.as<float>();
+    const bool af = l == 0 && x_f32;
+    if (af) {
+      g.Af = x_f32;
+      g.lda = net.dims[0];
+    }
+    TimedLaunch tl("mlp_gemm", s);
+    if (l + 1 < net.L)
+      af ? gemm_nt<NT_HIDDEN, true>(g, net.E, s) : gemm_nt<NT_HIDDEN>(g, net.E, s);
+    else
+      af ? gemm_nt<NT_OUT, true>(g, net.E, s) : gemm_nt<NT_OUT>(g, net.E, s);
+  }
+}
+
+int loss_tiles(const Mlp& net, int B) { return net.pd[net.L] / TN * (pad64(B) / TM); }
+
+// Adam's numbers of one step; null pointers elsewhere mean gradients only.
+struct AdamStep {
+  float lr, b1, b2, eps, bc1, bc2;
+};
+
+// One training pass of every member over the minibatch whose inputs are in
+// xb/xT: forward, loss and its gradient against T (rows idx, or 0..B-1), then
+// per layer, from the last, the input gradient and the weight gradient.  With
+// adam the weight gradients go straight into the update (the layer's old
+// weights were read by the input gradient queued before it), else to g.
+// lossp: [E][loss_tiles] sums of squares.
+void train_pass(Mlp& net, int B, const float* T, const int32_t* idx, double* lossp, const AdamStep* adam,
+                hipStream_t s) {
+  const int L = net.L, rows = pad64(B);
+  for (int l = 0; l < L; ++l) {
+    NtArgs g{};
+    g.A = l ? net.hb[l - 1].as<uint16_t>() : net.xb.as<uint16_t>();
+    g.lda = g.K = net.pd[l];
+    g.a_z = l ? (int64_t)rows * net.pd[l] : 0;
+    g.B = net.wb.as<uint16_t>() + net.wbo[l];
+    g.ldb = net.pd[l];
+    g.b_z = net.PB;
+    g.M = B;
+    g.N = net.dims[l + 1];
+    g.mp = rows;
+    g.np = net.pd[l + 1];
     g.bias = net.w.as<float>() + net.b_off[l];
     g.bias_z = net.P;
     TimedLaunch tl("mlp_gemm", s);
-    if (l + 1 < net.L) {
-      g.Cf = inference ? nullptr : net.zf[l].as<float>();
-      g.Cb = net.hb[l].as<uint16_t>();
-      gemm_fwd<EPI_BIAS_GELU>(g, net.E, s);
-      x = net.hb[l].as<uint16_t>();
-      x_z = (int64_t)B * outd;
+    if (l + 1 < L) {
+      g.z = net.zf[l].as<float>();
+      g.C = net.hb[l].as<uint16_t>();
+      g.CT = net.hT[l].as<uint16_t>();
+      gemm_nt<NT_GELU>(g, net.E, s);
     } else {
-      g.Cf = net.out.as<float>();
-      gemm_fwd<EPI_BIAS>(g, net.E, s);
+      g.C = net.dz[l].as<uint16_t>();
+      g.CT = net.dzT[l].as<uint16_t>();
+      g.T = T;
+      g.idx = idx;
+      g.lossp = lossp;
+      gemm_nt<NT_MSE>(g, net.E, s);
+    }
+  }
+  for (int l = L - 1; l >= 0; --l) {
+    if (l > 0) {
+      // dZ_{l-1}[b][i] = (sum_o dZ[b][o] W[o][i]) * gelu'(Z_{l-1}[b][i])
+      NtArgs g{};
+      g.A = net.dz[l].as<uint16_t>();
+      g.lda = g.K = net.pd[l + 1];
+      g.a_z = (int64_t)rows * net.pd[l + 1];
+      g.B = net.wbT.as<uint16_t>() + net.wbo[l];
+      g.ldb = net.pd[l + 1];
+      g.b_z = net.PB;
+      g.M = B;
+      g.N = net.dims[l];
+      g.mp = rows;
+      g.np = net.pd[l];
+      g.z = net.zf[l - 1].as<float>();
+      g.C = net.dz[l - 1].as<uint16_t>();
+      g.CT = net.dzT[l - 1].as<uint16_t>();
+      TimedLaunch tl("mlp_gemm", s);
+      gemm_nt<NT_DGELU>(g, net.E, s);
+    }
+    // dW[o][i] = sum_b dZ[b][o] X[b][i]
+    NtArgs g{};
+    g.A = net.dzT[l].as<uint16_t>();
+    g.lda = g.ldb = g.K = rows;
+    g.a_z = (int64_t)rows * net.pd[l + 1];
+    g.B = l ? net.hT[l - 1].as<uint16_t>() : net.xT.as<uint16_t>();
+    g.b_z = l ? (int64_t)rows * net.pd[l] : 0;
+    g.M = net.dims[l + 1];
+    g.N = net.dims[l];
+    g.mp = net.pd[l + 1];
+    g.np = net.pd[l];
+    g.p_z = net.P;
+    g.b_off = net.b_off[l] - net.w_off[l];
+    if (adam) {
+      g.w = net.w.as<float>() + net.w_off[l];
+      g.m = net.m.as<float>() + net.w_off[l];
+      g.v = net.v.as<float>() + net.w_off[l];
+      g.wb = net.wb.as<uint16_t>() + net.wbo[l];
+      g.wbT = net.wbT.as<uint16_t>() + net.wbo[l];
+      g.wb_z = net.PB;
+      g.lr = adam->lr;
+      g.b1 = adam->b1;
+      g.b2 = adam->b2;
+      g.eps = adam->eps;
+      g.bc1 = adam->bc1;
+      g.bc2 = adam->bc2;
+      TimedLaunch tl("mlp_adam", s);
+      gemm_nt<NT_ADAM>(g, net.E, s);
+    } else {
+      g.g = net.g.as<float>() + net.w_off[l];
+      TimedLaunch tl("mlp_gemm", s);
+      gemm_nt<NT_GRAD>(g, net.E, s);
     }
   }
 }
 
-// gradients of the mean-squared error against yb into g; loss per member
-void backward(Mlp& net, int B, hipStream_t s) {
-  const int L = net.L;
-  const int64_t BN = (int64_t)B * net.dims[L];
-  HIP_CHECK(hipMemsetAsync(net.loss.p, 0, net.E * 8, s));
-  hipLaunchKernelGGL(mse_grad_kernel, dim3(blocks_for(BN, 256), net.E), dim3(256), 0, s, net.out.as<float>(),
-                     net.yb.as<float>(), BN, net.dz[L - 1].as<uint16_t>(), net.loss.as<double>());
+// Minibatch inputs of X (rows idx, or 0..B-1) into xb and xT.
+void gather_batch(Mlp& net, const float* X, const int32_t* idx, int B, hipStream_t s) {
+  const int rows = pad64(B);
+  hipLaunchKernelGGL(gather_kernel, dim3(blocks_for(rows, 64)), dim3(64), 0, s, X, net.dims[0], idx, B, rows,
+                     net.pd[0], net.xb.as<uint16_t>(), net.xT.as<uint16_t>());
   HIP_CHECK(hipGetLastError());
-  for (int l = L - 1; l >= 0; --l) {
-    const int in = net.dims[l], outd = net.dims[l + 1];
-    const uint16_t* dZ = net.dz[l].as<uint16_t>();
-    const uint16_t* X = l > 0 ? net.hb[l - 1].as<uint16_t>() : net.xb.as<uint16_t>();
-    const int64_t x_z = l > 0 ? (int64_t)B * in : 0;
-    {
-      // dW[o][i] = sum_b dZ[b][o] X[b][i]
-      GemmArgs g{};
-      g.A = dZ;
-      g.lda = outd;
-      g.a_z = (int64_t)B * outd;
-      g.B = X;
-      g.ldb = in;
-      g.b_z = x_z;
-      g.M = outd;
-      g.N = in;
-      g.K = B;
-      g.Cf = net.g.as<float>() + net.w_off[l];
-      g.ldc = in;
-      g.c_z = net.P;
-      TimedLaunch tl("mlp_gemm", s);
-      gemm<false, false, EPI_F32>(g, net.E, s);
-    }
-    hipLaunchKernelGGL(bias_grad_kernel, dim3(blocks_for(outd, 256), net.E), dim3(256), 0, s, dZ, B, outd,
-                       (int64_t)B * outd, net.g.as<float>() + net.b_off[l], net.P);
-    HIP_CHECK(hipGetLastError());
-    if (l > 0) {
-      // dZ_{l-1}[b][i] = (sum_o dZ[b][o] W[o][i]) * gelu'(Z_{l-1}[b][i])
-      GemmArgs g{};
-      g.A = dZ;
-      g.lda = outd;
-      g.a_z = (int64_t)B * outd;
-      g.B = net.wb.as<uint16_t>() + net.w_off[l];
-      g.ldb = in;
-      g.b_z = net.P;
-      g.M = B;
-      g.N = in;
-      g.K = outd;
-      g.Cb = net.dz[l - 1].as<uint16_t>();
-      g.ldc = in;
-      g.c_z = (int64_t)B * in;
-      g.aux = net.zf[l - 1].as<float>();
-      TimedLaunch tl("mlp_gemm", s);
-      gemm<true, false, EPI_DGELU>(g, net.E, s);
-    }
-  }
 }
 
 // x into the mapped input buffer; convert_batch_input launches the
@@ -757,7 +758,7 @@ void stage_batch_input(Mlp& net, const float* x_host, int B) {
 void convert_batch_input(Mlp& net, int B, hipStream_t s) {
   const int64_t n = (int64_t)B * net.dims[0];
   hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, static_cast<const float*>(net.xin.d),
-                     n, net.xb.as<uint16_t>());
+                     n, net.dims[0], net.pd[0], net.xb.as<uint16_t>());
   HIP_CHECK(hipGetLastError());
 }
 
@@ -782,18 +783,27 @@ Mlp* mlp_create(int E, int L, const int32_t* dims, int max_batch) {
   }
   // members start 16-element aligned so every BF16 row load stays aligned
   net->P = (off + 15) / 16 * 16;
+  for (int l = 0; l <= L; ++l) net->pd.push_back(pad64(dims[l]));
+  for (int l = 0; l < L; ++l) {
+    net->wbo.push_back(net->PB);
+    net->PB += (int64_t)net->pd[l + 1] * net->pd[l];
+  }
   const int64_t tot = (int64_t)E * net->P;
   net->w.reserve(tot * 4);
-  net->wb.reserve(tot * 2);
+  net->wb.reserve((size_t)E * net->PB * 2);
+  net->wbT.reserve((size_t)E * net->PB * 2);
   net->g.reserve(tot * 4);
   net->m.reserve(tot * 4);
   net->v.reserve(tot * 4);
   HIP_CHECK(hipMemset(net->w.p, 0, tot * 4));
-  HIP_CHECK(hipMemset(net->wb.p, 0, tot * 2));
+  HIP_CHECK(hipMemset(net->wb.p, 0, (size_t)E * net->PB * 2));
+  HIP_CHECK(hipMemset(net->wbT.p, 0, (size_t)E * net->PB * 2));
   HIP_CHECK(hipMemset(net->g.p, 0, tot * 4));
   HIP_CHECK(hipMemset(net->m.p, 0, tot * 4));
   HIP_CHECK(hipMemset(net->v.p, 0, tot * 4));
-  alloc_acts(*net, std::max(max_batch, 1));
+  net->max_batch = std::max(max_batch, 1);
+  alloc_acts(*net, net->max_batch, nullptr);
+  HIP_CHECK(hipStreamSynchronize(nullptr));
   return net.release();
 }
 
@@ -814,9 +824,13 @@ void mlp_get_params(Mlp& net, float* params, hipStream_t s) {
 void mlp_set_params(Mlp& net, const float* params, hipStream_t s) {
   const int64_t tot = (int64_t)net.E * net.P;
   HIP_CHECK(hipMemcpyAsync(net.w.p, params, tot * 4, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(to_bf16_kernel, dim3(blocks_for(tot, 256)), dim3(256), 0, s, net.w.as<float>(), tot,
-                     net.wb.as<uint16_t>());
-  HIP_CHECK(hipGetLastError());
+  for (int l = 0; l < net.L; ++l) {
+    const int64_t n = (int64_t)net.pd[l + 1] * net.pd[l];
+    hipLaunchKernelGGL(pack_weights_kernel, dim3(blocks_for(n, 256), net.E), dim3(256), 0, s,
+                       net.w.as<float>() + net.w_off[l], net.P, net.dims[l + 1], net.dims[l], net.pd[l + 1], net.pd[l],
+                       net.wb.as<uint16_t>() + net.wbo[l], net.wbT.as<uint16_t>() + net.wbo[l], net.PB);
+    HIP_CHECK(hipGetLastError());
+  }
   HIP_CHECK(hipMemsetAsync(net.m.p, 0, tot * 4, s));
   HIP_CHECK(hipMemsetAsync(net.v.p, 0, tot * 4, s));
   stream_sync(s);
@@ -824,9 +838,9 @@ void mlp_set_params(Mlp& net, const float* params, hipStream_t s) {
 }
 
 void mlp_forward(Mlp& net, const float* x_host, int B, float* y_host, hipStream_t s) {
-  alloc_acts(net, B);
+  alloc_acts(net, B, s);
   upload_batch_input(net, x_host, B, s);
-  forward(net, B, s, nullptr, true);  // the network's outputs as predictions form them
+  forward(net, B, s);  // the network's outputs as predictions form them
   d2h(y_host, net.out.p, (size_t)net.E * B * net.dims[net.L], s);
   stream_sync(s);
 }
@@ -876,10 +890,10 @@ bool launch_stats_reg(int K, int E, int B, const float* y, int D, const double* 
 // Conversion, forward pass and ensemble statistics of B staged samples.
 void enqueue_predict(Mlp& net, int B, double scale, bool with_target, bool with_mean, hipStream_t s) {
   if (net.dims[0] % 8 == 0) {
-    forward(net, B, s, static_cast<const float*>(net.xin.d), true);  // inputs read from the mapped buffer
+    forward(net, B, s, static_cast<const float*>(net.xin.d));  // inputs read from the mapped buffer
   } else {
     convert_batch_input(net, B, s);
-    forward(net, B, s, nullptr, true);
+    forward(net, B, s);
   }
   const int D = net.dims[net.L];
   const double* tgt = with_target ? net.st.as<double>() : nullptr;
@@ -902,17 +916,10 @@ hipGraphExec_t predict_graph(Mlp& net, int B, double scale, bool with_target, bo
                                 (uintptr_t)net.xin.d, (uintptr_t)net.sout.d, (uintptr_t)net.smean.p,
                                 (uintptr_t)net.sw.p, (uintptr_t)net.st.p, (uintptr_t)net.xb.p,
                                 (uintptr_t)net.wb.p, (uintptr_t)net.w.p, (uintptr_t)net.out.p};
-  for (int l = 0; l < net.L; ++l) {
-    key.push_back((uintptr_t)net.zf[l].p);
-    key.push_back((uintptr_t)net.hb[l].p);
-  }
+  for (int l = 0; l < net.L; ++l) key.push_back((uintptr_t)net.hb[l].p);
   for (const auto& g : net.graphs)
     if (g.key == key) return g.exec;
   if (!net.cap) HIP_CHECK(hipStreamCreateWithFlags(&net.cap, hipStreamNonBlocking));
-  fwd_attr<EPI_BIAS_GELU>();  // kernel attributes are set outside the capture
-  fwd_attr<EPI_BIAS>();
-  fwd_attr<EPI_BIAS_GELU, true>();
-  fwd_attr<EPI_BIAS, true>();
   HIP_CHECK(hipStreamBeginCapture(net.cap, hipStreamCaptureModeThreadLocal));
   hipGraph_t graph = nullptr;
   try {
@@ -946,7 +953,7 @@ void mlp_predict(Mlp& net, const float* x_host, int B, const double* w_host, dou
 
 void mlp_predict_begin(Mlp& net, const float* x_host, int B, const double* w_host, double scale,
                        const double* target_host, double* mean_host, hipStream_t s) {
-  alloc_acts(net, B);
+  alloc_acts(net, B, s);
   stage_batch_input(net, x_host, B);
   const int D = net.dims[net.L];
   upload_on_change(net.sw, net.sw_host, w_host, D, s);
@@ -971,12 +978,19 @@ void mlp_predict_end(Mlp& net, int B, bool with_target, double* dis_host, double
 
 void mlp_gradients(Mlp& net, const float* x_host, const float* y_host, int B, float* g_host, double* loss,
                    hipStream_t s) {
-  alloc_acts(net, B);
-  upload_batch_input(net, x_host, B, s);
-  h2d(net.yb, y_host, (size_t)B * net.dims[net.L], s);
+  alloc_train(net, B, s);
+  stage_batch_input(net, x_host, B);
+  DevBuf yb, lossp;
+  h2d(yb, y_host, (size_t)B * net.dims[net.L], s);
+  const int tiles = loss_tiles(net, B);
+  lossp.reserve((size_t)net.E * tiles * 8);
+  net.loss.reserve(net.E * 8);
   HIP_CHECK(hipMemsetAsync(net.g.p, 0, (size_t)net.E * net.P * 4, s));
-  forward(net, B, s);
-  backward(net, B, s);
+  gather_batch(net, static_cast<const float*>(net.xin.d), nullptr, B, s);
+  train_pass(net, B, yb.as<float>(), nullptr, lossp.as<double>(), nullptr, s);
+  hipLaunchKernelGGL(loss_sum_kernel, dim3(net.E), dim3(64), 0, s, lossp.as<double>(), tiles,
+                     (double)B * net.dims[net.L], net.loss.as<double>());
+  HIP_CHECK(hipGetLastError());
   if (g_host) d2h(g_host, net.g.p, (size_t)net.E * net.P, s);
   if (loss) d2h(loss, net.loss.p, net.E, s);
   stream_sync(s);
@@ -991,26 +1005,23 @@ void mlp_set_data(Mlp& net, const float* X, const float* Y, int64_t n, hipStream
 
 void mlp_train(Mlp& net, const int32_t* batches, int steps, int B, float lr, float b1, float b2, float eps,
                double* losses, hipStream_t s) {
-  alloc_acts(net, B);
-  DevBuf didx;
+  alloc_train(net, B, s);
+  DevBuf didx, lossp, lbuf;
   h2d(didx, batches, (size_t)steps * B, s);
-  const int64_t tot = (int64_t)net.E * net.P;
-  DevBuf lbuf;
-  lbuf.reserve((size_t)std::max(steps, 1) * net.E * 8);
+  const int tiles = loss_tiles(net, B);
+  const int n_loss = std::max(steps, 1) * net.E;
+  lossp.reserve((size_t)n_loss * tiles * 8);
+  lbuf.reserve((size_t)n_loss * 8);
   for (int it = 0; it < steps; ++it) {
-    hipLaunchKernelGGL(gather_kernel, dim3(B), dim3(256), 0, s, net.dX.as<float>(), net.dims[0], net.dY.as<float>(),
-                       net.dims[net.L], didx.as<int32_t>() + (size_t)it * B, B, net.xb.as<uint16_t>(),
-                       net.yb.as<float>());
-    HIP_CHECK(hipGetLastError());
-    forward(net, B, s);
-    backward(net, B, s);
-    HIP_CHECK(hipMemcpyAsync(lbuf.as<double>() + (size_t)it * net.E, net.loss.p, net.E * 8, hipMemcpyDeviceToDevice,
-                             s));
+    const int32_t* idx = didx.as<int32_t>() + (size_t)it * B;
+    gather_batch(net, net.dX.as<float>(), idx, B, s);
     ++net.step;
-    const float bc1 = 1.0f - powf(b1, (float)net.step), bc2 = 1.0f - powf(b2, (float)net.step);
-    TimedLaunch tl("mlp_adam", s);
-    hipLaunchKernelGGL(adam_kernel, dim3(blocks_for(tot, 256)), dim3(256), 0, s, net.w.as<float>(), net.g.as<float>(),
-                       net.m.as<float>(), net.v.as<float>(), net.wb.as<uint16_t>(), tot, lr, b1, b2, eps, bc1, bc2);
+    const AdamStep adam{lr, b1, b2, eps, 1.0f - powf(b1, (float)net.step), 1.0f - powf(b2, (float)net.step)};
+    train_pass(net, B, net.dY.as<float>(), idx, lossp.as<double>() + (size_t)it * net.E * tiles, &adam, s);
+  }
+  if (steps > 0) {
+    hipLaunchKernelGGL(loss_sum_kernel, dim3(steps * net.E), dim3(64), 0, s, lossp.as<double>(), tiles,
+                       (double)B * net.dims[net.L], lbuf.as<double>());
     HIP_CHECK(hipGetLastError());
   }
   if (losses) d2h(losses, lbuf.p, (size_t)steps * net.E, s);
