@@ -14,8 +14,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libimped.so")
-SOURCES = ["krylov.hip", "lanczos_reg_real.hip", "lanczos_reg_cplx.hip", "engine.hip", "mlp.hip", "apply.hip", "prims.hip",
-           "vecops.hip", "walkers.hip"]
+SOURCES = ["eigen_reg_cplx.hip", "eigen_reg_real.hip", "lanczos_reg_cplx.hip", "lanczos_reg_real.hip", "krylov.hip",
+           "engine.hip", "mlp.hip", "apply.hip", "prims.hip", "vecops.hip", "walkers.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "-O3",

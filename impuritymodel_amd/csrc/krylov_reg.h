@@ -26,6 +26,8 @@
 
 namespace imped {
 
+struct EigenArgs;
+
 struct LanczosArgs {
   const int64_t* row_base;
   const int64_t* chain_n;
@@ -66,5 +68,11 @@ constexpr int kRegClasses = 7;
 // vector; H real) run in the real launch, the others in the complex one.
 void launch_lanczos_reg_real(const LanczosArgs& a, unsigned nb, int n_cu, int groups, hipStream_t s);
 void launch_lanczos_reg_cplx(const LanczosArgs& a, unsigned nb, int n_cu, int groups, hipStream_t s);
+
+// The eigensolver on the same basis: nb chains of at most a.nmax <= kRegMaxN
+// rows; with test nothing is launched and the result says whether the launch's
+// arrays fit the LDS (for every number of groups when for 4).
+bool launch_eigen_reg_real(const EigenArgs& a, unsigned nb, int n_cu, int groups, bool test, hipStream_t s);
+bool launch_eigen_reg_cplx(const EigenArgs& a, unsigned nb, int n_cu, int groups, bool test, hipStream_t s);
 
 }  // namespace imped

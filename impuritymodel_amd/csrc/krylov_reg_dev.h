@@ -93,7 +93,7 @@ struct RegBasis {
   T* vg;        // memory: vector l at vg + l*n
   double* dotp;  // LDS [NQ][lcap * D * G]: dots of wave q's rows, by group and local index
   double* cw;    // LDS [W][lcap * D]: this wave's coefficients
-  T* upd;       // LDS [G][NQ*64*R]: updates of the groups (G > 1)
+  T* upd;       // LDS [G][NQ*64*R]: the groups' updates, and parts of H v (G > 1)
   double* red;  // LDS [3][W]
   int lcap;     // local vectors per group, a multiple of B
 
@@ -258,6 +258,34 @@ struct RegBasis {
     return t;
   }
 
+  // (yr, yi) <- the groups' parts of H v summed; returns Re <v, H v>.  One
+  // barrier: the parts and each wave's share of the product go to LDS together.
+  __device__ __forceinline__ double product(const T (&v)[R], double (&yr)[R], double (&yi)[R]) {
+    double p = 0.0;
+#pragma unroll
+    for (int r = 0; r < R; ++r) p += re1(v[r]) * yr[r] + im1(v[r]) * yi[r];
+    if constexpr (G == 1) return row_sum(p, 2);
+    p = wave_sum(p);
+    if (lane == 0) red[2 * W + wave] = p;
+#pragma unroll
+    for (int r = 0; r < R; ++r) set1(upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane], yr[r], yi[r]);
+    __syncthreads();
+    p = 0.0;
+#pragma unroll
+    for (int k = 0; k < W; ++k) p += red[2 * W + k];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      yr[r] = yi[r] = 0.0;
+#pragma unroll
+      for (int k = 0; k < G; ++k) {
+        const T t = upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
+        yr[r] += re1(t);
+        yi[r] += im1(t);
+      }
+    }
+    return p;
+  }
+
   // One classical Gram-Schmidt pass of w against vectors 0..m-1; *pw receives
   // |w|^2 before the pass.
   __device__ __forceinline__ void pass(int m, T (&w)[R], double* pw) {
@@ -343,11 +371,53 @@ struct RegBasis {
       }
     }
   }
+
+  // x = sum over l < m of y[l] v_l (real y; the same sum in every group)
+  __device__ __forceinline__ void combine(int m, const double* y, T (&out)[R]) {
+    const int nl = __builtin_amdgcn_readfirstlane((m - g + G - 1) / G);
+    double ur[R], ui[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) ur[r] = ui[r] = 0.0;
+    auto add = [&](double c, int r, const T& t) __attribute__((always_inline)) {
+      ur[r] += c * re1(t);
+      if constexpr (!reg_real_v<T>) ui[r] += c * im1(t);
+    };
+    static_for<S>([&](auto s) __attribute__((always_inline)) {
+      if (s < nl)
+        static_for<R>([&](auto r) __attribute__((always_inline)) { add(y[s * G + g], r, slot<s, r>()); });
+    });
+    const int n1 = nl < S + kl ? nl : S + kl;
+    for (int li = S; li < n1; ++li)
+#pragma unroll
+      for (int r = 0; r < R; ++r) add(y[li * G + g], r, vl[(size_t)((li - S) * G + g) * n + row[r]]);
+#pragma unroll 4
+    for (int li = S + kl; li < nl; ++li)
+#pragma unroll
+      for (int r = 0; r < R; ++r) add(y[li * G + g], r, vg[(size_t)(li * G + g) * n + row[r]]);
+    if constexpr (G > 1) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) set1(upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane], ur[r], ui[r]);
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        ur[r] = ui[r] = 0.0;
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+          const T t = upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
+          ur[r] += re1(t);
+          ui[r] += im1(t);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) set1(out[r], on[r] ? ur[r] : 0.0, on[r] ? ui[r] : 0.0);
+  }
 };
 
-// The rows of H of one thread: up to HR entries of each in registers, the
-// rest read from memory.
-template <int R, class T>
+// The rows of H of one thread: group g takes entries g, g + G, ... of each row,
+// up to HR of them in registers, the rest read from memory (the groups'
+// products of a row meet in RegBasis::product).
+template <int W, int G, int R, class T>
 struct RegRows {
   static constexpr int HR = reg_row_entries<R, T>();
   T h[R][HR ? HR : 1];
@@ -355,7 +425,7 @@ struct RegRows {
   int cnt_wave[R];
   int64_t rest[R], end[R];
 
-  __device__ __forceinline__ void load(const int64_t* rowptr, const int32_t* col, const double2* val,
+  __device__ __forceinline__ void load(const int64_t* rowptr, const int32_t* col, const double2* val, int g,
                                        const int (&row)[R], const bool (&on)[R]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -363,26 +433,27 @@ struct RegRows {
       rest[r] = end[r] = 0;
       int64_t e0 = 0;
       if (on[r]) {
-        e0 = rowptr[row[r]];
+        e0 = rowptr[row[r]] + g;
         end[r] = rowptr[row[r] + 1];
-        cnt = (int)(end[r] - e0 < HR ? end[r] - e0 : HR);
-        rest[r] = e0 + cnt;
+        const int64_t mine = end[r] > e0 ? (end[r] - e0 + G - 1) / G : 0;
+        cnt = (int)(mine < HR ? mine : HR);
+        rest[r] = e0 + (int64_t)cnt * G;
       }
 #pragma unroll
       for (int k = 0; k < HR; ++k) {
         set1(h[r][k], 0.0, 0.0);
         c[r][k] = 0;
         if (k < cnt) {
-          const double2 t = val[e0 + k];
+          const double2 t = val[e0 + (int64_t)k * G];
           set1(h[r][k], t.x, t.y);
-          c[r][k] = col[e0 + k];
+          c[r][k] = col[e0 + (int64_t)k * G];
         }
       }
       cnt_wave[r] = wave_max_int(cnt);
     }
   }
 
-  // row r of H x (x in LDS)
+  // this group's part of row r of H x (x in LDS)
   __device__ __forceinline__ void apply(int r, const int32_t* col, const double2* val, const T* x, double* yr,
                                         double* yi) const {
     double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
@@ -406,18 +477,18 @@ struct RegRows {
         add(bx, by, h[r][k0 + 3], t[3]);
       }
     // four entries per round trip (indices past the row clamped, their products skipped)
-    for (int64_t e = rest[r]; e < end[r]; e += 4) {
+    for (int64_t e = rest[r]; e < end[r]; e += 4 * G) {
       T hh[4], t[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int64_t k = e + u < end[r] ? e + u : end[r] - 1;
+        const int64_t k = e + u * G < end[r] ? e + u * G : end[r] - 1;
         const double2 z = val[k];
         set1(hh[u], z.x, z.y);
         t[u] = x[col[k]];
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (e + u < end[r]) add(ax, ay, hh[u], t[u]);
+        if (e + u * G < end[r]) add(ax, ay, hh[u], t[u]);
     }
     *yr = ax + bx;
     *yi = ay + by;

@@ -47,8 +47,8 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs
   Basis b;
   b.init(n, K, a.kl, reinterpret_cast<double*>(lds) + ((size_t)a.nmax * Basis::D + 1) / 2 * 2,
          reinterpret_cast<T*>(a.vstore + (size_t)a.K * base));
-  RegRows<R, T> h;
-  h.load(a.rowptr + base, a.col, a.val, b.row, b.on);
+  RegRows<NQ * G, G, R, T> h;
+  h.load(a.rowptr + base, a.col, a.val, b.g, b.row, b.on);
   T w[R], vp[R];  // the residual; the latest basis vector
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -74,16 +74,15 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs
   for (int j = 0;; ++j) {
     // v_j = w / beta; y = H v_j; alpha_j = Re <v_j, y>
     T v[R];
-    double yr[R], yi[R], p = 0.0;
+    double yr[R], yi[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       set1(v[r], re1(w[r]) * sc, im1(w[r]) * sc);
       h.apply(r, a.col, a.val, xs, &yr[r], &yi[r]);
       yr[r] *= sc;
       yi[r] *= sc;
-      p += re1(v[r]) * yr[r] + im1(v[r]) * yi[r];
     }
-    const double al = b.row_sum(p, 2);
+    const double al = b.product(v, yr, yi);
     if (threadIdx.x == 0) alpha[j] = al;
     if (j + 1 == K) break;
     b.store(j, v);
@@ -94,7 +93,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs
     }
     // full reorthogonalization against v_0..v_j; a second pass when the
     // first removed more than half of |w|^2
-    double p1, pw = 0.0;
+    double p, p1, pw = 0.0;
     for (int it = 0;; ++it) {
       double before;
       b.pass(j + 1, w, &before);
