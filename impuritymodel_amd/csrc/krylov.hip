@@ -496,11 +496,13 @@ struct OrthEstimate {
 
 // LW: the tridiagonal and the Ritz work arrays live in LDS (a compile-time
 // choice, so every access to them is an LDS instruction), else in memory.
-// The basis is in memory (chains beyond the register kernels): Gram-Schmidt
-// passes, each reading it twice, are made only in the steps where the
-// estimated inner products ask for one (OrthEstimate's recurrence and level,
-// one thread per basis vector), with dgks off two in every step.  Measured, 23
-// real chains of 190 to 1770 rows, 132 steps at most: 5.5 -> 2.9 ms.
+// The basis is in memory (chains beyond the register kernels) and every step
+// makes its Gram-Schmidt pass, read by one CU: what bounds it.  Passes only where
+// OrthEstimate asks for one take 23 real chains of 190 to 1770 rows (132 steps at
+// most) from 5.5 to 2.9 ms, but the eigenvectors' last bits then differ, and the
+// unconverged plain recurrences that start from them show it: 150 steps on 900
+// rows scatter by 1e-3 to 3.5e-3 of a resonant map's peak between eigenvectors
+// that agree to 1e-12, so the chains of this size keep the vectors they had.
 template <int BT, class T, bool LW>
 __global__ __launch_bounds__(BT) void eigen_kernel(EigenArgs a) {
   __shared__ double red[BT / 64];
@@ -553,15 +555,6 @@ __global__ __launch_bounds__(BT) void eigen_kernel(EigenArgs a) {
     pivb = a.tpiv + (size_t)c * nev * ms;
   }
   T* w = reinterpret_cast<T*>(a.wbuf) + base;
-  // estimated inner products of v_j and of v_{j-1} with the basis, and work
-  double* om[3];
-  if constexpr (LW)
-    om[0] = reinterpret_cast<double*>(pivb + ((size_t)nev * L + 1) / 2 * 2);
-  else
-    om[0] = a.om + (size_t)c * 3 * (ms + 2);
-  om[1] = om[0] + ys + 2;
-  om[2] = om[1] + ys + 2;
-  bool again = false;  // the step after a pass
   // seeded random start vector (real when T is real)
   {
     auto start = [&](T* V0) {
@@ -641,37 +634,14 @@ __global__ __launch_bounds__(BT) void eigen_kernel(EigenArgs a) {
       p0 = three_term<BT, T>(a, base, n, VG, VG, false, 0.0, w, red, &al);
     else
       p0 = three_term<BT, T>(a, base, n, VG + (size_t)j * n, VG + (size_t)(j - 1) * n, true, bprev, w, red, &al);
-    bool pass = again || !a.dgks;
-    {
-      const double bt = sqrt(p0);
-      double worst = bt > 0.0 ? 0.0 : INFINITY;
-      const double *wj = om[j % 3], *wo = om[(j + 2) % 3];
-      double* wn = om[(j + 1) % 3];
-      for (int k = threadIdx.x; k < j; k += BT) {
-        double t = sb[k] * (k + 1 < j ? wj[k + 1] : 1.0) + (sa[k] - al) * wj[k] - bprev * (k + 1 < j ? wo[k] : 1.0);
-        if (k > 0) t += sb[k - 1] * wj[k - 1];
-        t = (t + copysign(4.4e-16 * (sb[k] + bt), t)) / bt;
-        wn[k] = t;
-        worst = fmax(worst, fabs(t));
-      }
-      if (threadIdx.x == 0) {
-        const double t = 2.2e-16 * (fabs(al) + bt + bprev) / bt;
-        wn[j] = t;
-        worst = fmax(worst, t);
-      }
-      const bool over = __syncthreads_or(!(worst <= kOrthLevel)) != 0;
-      again = (over || again) && !again;
-      pass = pass || over;
-    }
-    double p1 = p0;
-    if (pass) {
+    // full reorthogonalization against V_0..V_j; a second pass when the first
+    // removed more than half of |w|^2 (Daniel-Gragg-Kaufman-Stewart), or in
+    // every step with dgks off
+    dots_basis<BT, T>(VG, j + 1, n, w, cl);
+    double p1 = update_basis<BT, T>(VG, j + 1, n, w, cl, red);
+    if (!a.dgks || p1 < 0.5 * p0) {
       dots_basis<BT, T>(VG, j + 1, n, w, cl);
       p1 = update_basis<BT, T>(VG, j + 1, n, w, cl, red);
-      if (!a.dgks || p1 < 0.5 * p0) {
-        dots_basis<BT, T>(VG, j + 1, n, w, cl);
-        p1 = update_basis<BT, T>(VG, j + 1, n, w, cl, red);
-      }
-      for (int k = threadIdx.x; k <= j; k += BT) om[(j + 1) % 3][k] = 2.2e-16;
     }
     if (threadIdx.x == 0) {
       alpha[j] = al;
@@ -1705,7 +1675,7 @@ struct KScratch {
   DevBuf ws, vstore, coef, ab, yk, tw, tpiv, voff, conv, wbuf, clist;
   DevBuf cf_alpha_tmp, cf_in, gout, sout;
   DevBuf fpart, fcpart, fcoef, fscal;
-  DevBuf sz, scz, sres, ssteps, eig_in, pure, om;
+  DevBuf sz, scz, sres, ssteps, eig_in, pure;
 };
 KScratch& kscratch() {
   static KScratch k;
@@ -2243,9 +2213,8 @@ void run_lanczos(const KrylovBatch& kb, const double2* v0, int K, int reorth, do
 }
 
 // Chains of up to this many rows are solved on the register kernels.  Beyond, the
-// basis no longer fits the CU and 1024 threads on a basis in memory with partial
-// reorthogonalization are faster (780 rows: 2.8 ms on the register kernel, below
-// 2.9 ms for a launch whose largest chain has 1770 rows).
+// basis no longer fits the CU's registers and LDS (780 rows, four per thread: 2.8 ms
+// on the register kernel).
 constexpr int64_t kEigenRegMaxN = 512;
 
 int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_t seed, double* evals,
@@ -2320,7 +2289,6 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
   sc.yk.reserve((size_t)C * nev * max_steps * 8);
   sc.tw.reserve((size_t)C * nev * 5 * max_steps * 8);
   sc.tpiv.reserve((size_t)C * nev * max_steps * 4);
-  sc.om.reserve((size_t)C * 3 * (max_steps + 2) * 8);
   EigenArgs a{};
   a.row_base = kb.row_base;
   a.chain_n = kb.chain_n;
@@ -2338,7 +2306,6 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
   a.yk = sc.yk.as<double>();
   a.tw = sc.tw.as<double>();
   a.tpiv = sc.tpiv.as<int>();
-  a.om = sc.om.as<double>();
   a.evals = evals;
   a.evecs = evecs;
   a.steps = steps;
@@ -2388,14 +2355,13 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
   size_t n_wide = 0;
   while (n_wide < order.size() && kb.h_n[order[n_wide]] > g_tuning.eigen_wave_max_n) ++n_wide;
   // LDS layout of a launch whose largest chain is order[first]: coefficients
-  // always, alpha/beta, the Ritz work arrays and the orthogonality estimates when
-  // they fit in 60 KiB (the 64 KiB per-workgroup limit less the kernel's static
-  // arrays)
+  // always, alpha/beta and the Ritz work arrays when they fit in 60 KiB (the
+  // 64 KiB per-workgroup limit less the kernel's static arrays)
   size_t shm = 0;
   auto layout = [&](size_t first) {
     const int L = (int)std::min<int64_t>(max_steps, kb.h_n[order[first]]);
     const size_t coef = (size_t)(L + 2) * sizeof(double2), ab = 2 * (size_t)L * 8;
-    const size_t work = (size_t)nev * 5 * L * 8 + ((size_t)nev * L + 1) / 2 * 8 + 3 * (size_t)(L + 2) * 8;
+    const size_t work = (size_t)nev * 5 * L * 8 + ((size_t)nev * L + 1) / 2 * 8;
     a.lstride = L;
     a.lds_work = coef + ab + work <= 60 * 1024;
     shm = coef + (a.lds_work ? ab + work : 0);

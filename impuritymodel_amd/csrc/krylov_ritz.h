@@ -180,9 +180,7 @@ struct EigenArgs {
   int check_start;   // no check before this many steps (except at the last step)
   int lstride;       // LDS arrays: Gram-Schmidt coefficients (lstride + 2), then, when lds_work = 1,
   int lds_work;      //   alpha/beta (2 lstride), per eigenvalue y (lstride), LU work (4 lstride) and
-                     //   pivots (lstride ints), and the orthogonality estimates (3 (lstride + 2));
-                     //   lstride >= every chain's steps
-  double* om;        // per chain: 3 (max_steps + 2) orthogonality estimates
+                     //   pivots (lstride ints); lstride >= every chain's steps
   int kl;            // register kernels: vectors kept in LDS per group of waves
   int nmax;          //   and rows of the launch's largest chain
 };

@@ -1,5 +1,5 @@
 """Eigensolver on the register-resident basis (chains of up to 512 rows) and on
-the basis in memory with passes only where needed (larger chains), against numpy
+the basis in memory (larger chains), against numpy
 at the edges of the launch classes, real and complex, alone and in batches that
 change the number of waves per chain.
 
