@@ -14,10 +14,10 @@
 // the operator dict's order, the order in which applyOp adds them.
 //
 // A wave handles 64 sources of one model, so the group/term loops are
-// wave-uniform.  The wave copies its model's group and term tables into its
-// own LDS slice in chunks (coalesced vector loads, TERM_CHUNK terms and
-// GROUP_CHUNK groups at a time), and the loops read them from there: a term
-// then costs an LDS broadcast instead of a dependent scalar-cache miss.
+// wave-uniform.  The term table streams through the wave's registers: lane i
+// of a chunk holds term i's masks, value and sign data (one coalesced load
+// per 64 terms, the next chunk's in flight while this one is used), and a
+// term is broadcast to the wave by readlane.
 #include "kernels.h"
 
 namespace imped {
@@ -99,29 +99,67 @@ __device__ void hash_discover(const HashView& h, const CandView& c, int32_t chai
   }
 }
 
-constexpr int TERM_CHUNK = 128;  // terms per staged chunk (per wave)
-constexpr int GROUP_CHUNK = 64;  // groups per staged chunk (per wave)
-constexpr int RESTR_LDS = 16;    // restrictions kept in LDS (more are read from memory)
+constexpr int RESTR_LDS = 16;  // restrictions kept in LDS (more are read from memory)
 
-// LDS writes by some lanes of a wave, read by every lane of the same wave.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// Index of the first of group_term_off[lo..hi] that is >= x (hi if none is
+// smaller), searched 64 ways: every lane probes one position per round.
+__device__ __forceinline__ int group_at_term(const int32_t* gto, int lo, int hi, int x, int lane) {
+  while (lo < hi) {
+    const int step = (hi - lo + 63) >> 6;
+    const int idx = lo + lane * step;
+    const int below = __popcll(__ballot(idx < hi && gto[idx] < x));  // a prefix of the lanes
+    if (below == 0) break;
+    const int up = lo + below * step;
+    lo += (below - 1) * step + 1;
+    hi = up < hi ? up : hi;
+  }
+  return __builtin_amdgcn_readfirstlane(lo);
 }
 
+__device__ __forceinline__ uint64_t lane_u64(uint64_t v, int i) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, i);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), i);
+  return ((uint64_t)hi << 32) | lo;
+}
+__device__ __forceinline__ double lane_f64(double v, int i) {
+  return __longlong_as_double((long long)lane_u64((uint64_t)__double_as_longlong(v), i));
+}
+
+// 64 terms (one per lane) and 64 groups (one per lane) of the tables.
+template <int W>
+struct TermChunk {
+  uint64_t m[3 * W];
+  double2 c;
+  uint32_t meta;
+  __device__ __forceinline__ void load(const OpsView& o, int t, int t_end) {
+    if (t < t_end) {
+#pragma unroll
+      for (int w = 0; w < 3 * W; ++w) m[w] = o.term_masks[(size_t)t * 3 * W + w];
+      c = o.term_coef[t];
+      meta = o.term_meta[t];
+    }
+  }
+};
+
+// One wave per (64 sources, part of the model's groups): part p of a.split
+// takes the groups whose terms start in the p-th equal share of the model's
+// terms, and counts and offsets hold one value per (source, part), so the
+// entries of a source stay in group order whatever the split is.
+//
+// What bounds it: instruction issue of the walk over the terms, about 30 vector
+// instructions a term with a match and 10 without.  Measured on 1100-term models,
+// one launch: a few hundred sources 130 us with the terms in LDS and one wave per
+// task, 45 us so (the number operators are one group of hundreds of matching
+// terms, which stays with one wave); 3e6 sources of two words 1.6 to 1.1 ms.
 template <int W, int MODE, bool FILL>
 __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
-  __shared__ uint64_t l_mask[4][TERM_CHUNK * 3 * W];
-  __shared__ double2 l_coef[4][TERM_CHUNK];
-  __shared__ uint32_t l_meta[4][TERM_CHUNK];
-  __shared__ int32_t l_gto[4][GROUP_CHUNK + 1];
-  __shared__ uint64_t l_flip[4][GROUP_CHUNK * W];
   __shared__ uint64_t l_rmask[4][RESTR_LDS * W];
   __shared__ int32_t l_rlohi[4][RESTR_LDS * 2];
   const int lane = threadIdx.x & 63;
   const int wv = threadIdx.x >> 6;
-  const int64_t task_id = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;
+  const int64_t unit = (int64_t)blockIdx.x * (blockDim.x >> 6) + wv;
+  const int64_t task_id = unit / a.split;
+  const int part = __builtin_amdgcn_readfirstlane((int)(unit - task_id * a.split));
   if (task_id >= a.n_tasks) return;
   const WaveTask task = a.tasks[task_id];
   const int model = __builtin_amdgcn_readfirstlane(task.model);
@@ -139,21 +177,24 @@ __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
   }
   int64_t out = 0;
   int32_t cnt = 0;
-  if (FILL && active) out = a.offsets[src];
+  if (FILL && active) out = a.offsets[src * a.split + part];
 
   const OpsView& o = a.ops;
-  const int g0 = o.model_group_off[model];
-  const int g1 = o.model_group_off[model + 1];
+  int g0 = __builtin_amdgcn_readfirstlane(o.model_group_off[model]);
+  int g1 = __builtin_amdgcn_readfirstlane(o.model_group_off[model + 1]);
   const int r0 = o.model_restr_off[model];
   const int r1 = o.model_restr_off[model + 1];
-  const int t_end = o.group_term_off[g1];  // the model's terms end here
-  uint64_t* lm = l_mask[wv];
-  double2* lc = l_coef[wv];
-  uint32_t* lt = l_meta[wv];
-  int32_t* lg = l_gto[wv];
-  uint64_t* lf = l_flip[wv];
-  int gc0 = g0, gc1 = g0;  // staged groups [gc0, gc1)
-  int tc0 = 0, tc1 = 0;    // staged terms [tc0, tc1)
+  if (a.split > 1) {
+    const int tb = o.group_term_off[g0];
+    const int64_t T = o.group_term_off[g1] - tb;
+    const int lo = part > 0 ? group_at_term(o.group_term_off, g0, g1, tb + (int)(T * part / a.split), lane) : g0;
+    const int hi =
+        part + 1 < a.split ? group_at_term(o.group_term_off, g0, g1, tb + (int)(T * (part + 1) / a.split), lane) : g1;
+    g0 = lo;
+    g1 = hi;
+  }
+  int t = __builtin_amdgcn_readfirstlane(o.group_term_off[g0]);
+  const int t_end = __builtin_amdgcn_readfirstlane(o.group_term_off[g1]);  // this wave's terms end here
   const int nr = r1 - r0;
   const int nrl = nr < RESTR_LDS ? nr : RESTR_LDS;
   uint64_t* lrm = l_rmask[wv];
@@ -161,78 +202,85 @@ __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
   if (MODE != MODE_FIXED) {
     for (int i = lane; i < nrl * W; i += 64) lrm[i] = o.restr_mask[(size_t)r0 * W + i];
     for (int i = lane; i < nrl * 2; i += 64) lrl[i] = o.restr_lohi[2 * r0 + i];
+    // LDS writes by some lanes of the wave, read by every lane of it
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 
-  for (int g = g0; g < g1; ++g) {
-    if (g >= gc1) {
-      wave_lds_sync();  // every lane is done with the previous chunk
-      gc0 = g;
-      gc1 = g + GROUP_CHUNK < g1 ? g + GROUP_CHUNK : g1;
-      for (int i = lane; i <= gc1 - gc0; i += 64) lg[i] = o.group_term_off[gc0 + i];
-      for (int i = lane; i < (gc1 - gc0) * W; i += 64) lf[i] = o.group_flip[(size_t)gc0 * W + i];
-      wave_lds_sync();
+  TermChunk<W> cur{}, next{};
+  int tc0 = t;  // first term of the chunk in registers
+  cur.load(o, tc0 + lane, t_end);
+  next.load(o, tc0 + 64 + lane, t_end);
+  int gc0 = g0;  // first group in registers
+  int32_t gend = 0;
+  uint64_t gflip[W] = {};
+  auto load_groups = [&]() {
+    if (gc0 + lane < g1) {
+      gend = o.group_term_off[gc0 + lane + 1];
+#pragma unroll
+      for (int w = 0; w < W; ++w) gflip[w] = o.group_flip[(size_t)(gc0 + lane) * W + w];
     }
-    const int tb = lg[g - gc0];
-    const int te = lg[g - gc0 + 1];
+  };
+  load_groups();
+
+  for (int g = g0; g < g1; ++g) {
+    if (g - gc0 == 64) {
+      gc0 = g;
+      load_groups();
+    }
+    const int te = __builtin_amdgcn_readlane(gend, g - gc0);
     double2 acc = make_double2(0.0, 0.0);
     bool any = false;
     int first = 0;
     // one matching term: add its signed value (in term order)
-    auto take = [&](int t) {
-      const uint64_t* m = lm + (size_t)(t - tc0) * 3 * W;
-      const uint32_t meta = lt[t - tc0];
+    auto take = [&](int i) {
+      const uint32_t meta = __builtin_amdgcn_readlane(cur.meta, i);
       uint32_t par = meta & 1u;
 #pragma unroll
-      for (int w = 0; w < W; ++w) par ^= (uint32_t)__popcll(s[w] & m[2 * W + w]) & 1u;
-      const double2 c = lc[t - tc0];
+      for (int w = 0; w < W; ++w) par ^= (uint32_t)__popcll(s[w] & lane_u64(cur.m[2 * W + w], i)) & 1u;
+      const double cx = lane_f64(cur.c.x, i), cy = lane_f64(cur.c.y, i);
       if (par) {
-        acc.x -= c.x;
-        acc.y -= c.y;
+        acc.x -= cx;
+        acc.y -= cy;
       } else {
-        acc.x += c.x;
-        acc.y += c.y;
+        acc.x += cx;
+        acc.y += cy;
       }
       if (!any) first = (int)(meta >> 1);
       any = true;
     };
-    auto matches = [&](int t) {
-      const uint64_t* m = lm + (size_t)(t - tc0) * 3 * W;
-      bool ok = true;
+    auto matches = [&](int i) {
+      uint64_t diff = 0;
 #pragma unroll
-      for (int w = 0; w < W; ++w) ok = ok && ((s[w] & m[w]) == m[W + w]);
-      return ok;
+      for (int w = 0; w < W; ++w) diff |= (s[w] & lane_u64(cur.m[w], i)) ^ lane_u64(cur.m[W + w], i);
+      return diff == 0;
     };
-    for (int t = tb; t < te;) {
-      if (t >= tc1 || te > tc1) {
-        // stage from this term on (a group is staged whole when it fits a chunk)
-        if (t >= tc1 || (t == tb && te - tb <= TERM_CHUNK)) {
-          wave_lds_sync();
-          tc0 = t;
-          tc1 = t + TERM_CHUNK < t_end ? t + TERM_CHUNK : t_end;
-          for (int i = lane; i < (tc1 - tc0) * 3 * W; i += 64) lm[i] = o.term_masks[(size_t)tc0 * 3 * W + i];
-          for (int i = lane; i < tc1 - tc0; i += 64) {
-            lc[i] = o.term_coef[tc0 + i];
-            lt[i] = o.term_meta[tc0 + i];
-          }
-          wave_lds_sync();
-        }
+    while (t < te) {
+      if (t - tc0 == 64) {
+        tc0 = t;
+        cur = next;
+        next.load(o, tc0 + 64 + lane, t_end);
       }
-      const int tend = te < tc1 ? te : tc1;
-      // four mask tests per round trip, the matches taken in term order
-      for (; t + 4 <= tend; t += 4) {
-        const bool k0 = matches(t), k1 = matches(t + 1), k2 = matches(t + 2), k3 = matches(t + 3);
-        if (k0) take(t);
-        if (k1) take(t + 1);
-        if (k2) take(t + 2);
-        if (k3) take(t + 3);
+      const int iend = te - tc0 < 64 ? te - tc0 : 64;
+      int i = t - tc0;
+      // four mask tests at once, the matches taken in term order
+      for (; i + 4 <= iend; i += 4) {
+        const bool k0 = matches(i), k1 = matches(i + 1), k2 = matches(i + 2), k3 = matches(i + 3);
+        if (k0) take(i);
+        if (k1) take(i + 1);
+        if (k2) take(i + 2);
+        if (k3) take(i + 3);
       }
-      for (; t < tend; ++t)
-        if (matches(t)) take(t);
+      for (; i < iend; ++i)
+        if (matches(i)) take(i);
+      t = tc0 + iend;
     }
-    if (!(any && active)) continue;
+    if (__ballot(any && active) == 0) continue;
     uint64_t tgt[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) tgt[w] = s[w] ^ lf[(g - gc0) * W + w];
+    for (int w = 0; w < W; ++w) tgt[w] = s[w] ^ lane_u64(gflip[w], g - gc0);
+    if (!(any && active)) continue;
     bool keep = true;
     if (MODE != MODE_VECTOR) keep = abs2_ref(acc) >= a.weight_min;
     if (MODE != MODE_FIXED) {
@@ -277,13 +325,13 @@ __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
     }
     ++out;
   }
-  if (!FILL && active) a.counts[src] = cnt;
+  if (!FILL && active) a.counts[src * a.split + part] = cnt;
 }
 
 template <int W>
 static void launch_w(int mode, bool fill, const ApplyArgs& a, hipStream_t s) {
   const int threads = 256;
-  const unsigned blocks = blocks_for(a.n_tasks, threads / 64);
+  const unsigned blocks = blocks_for(a.n_tasks * a.split, threads / 64);
   if (a.n_tasks == 0) return;
   TimedLaunch tl(fill ? "apply_fill" : "apply_count", s);
 #define IMPED_LAUNCH(M, F) hipLaunchKernelGGL((apply_kernel<W, M, F>), dim3(blocks), dim3(threads), 0, s, a)
@@ -321,6 +369,12 @@ void launch_discover(int W, const uint64_t* keys, const int32_t* chain, int64_t 
   else
     hipLaunchKernelGGL(discover_kernel<2>, dim3(blocks_for(E, 256)), dim3(256), 0, s, keys, chain, E, h, c);
   HIP_CHECK(hipGetLastError());
+}
+
+int apply_split(int64_t n_tasks) {
+  int s = 1;
+  while (s < kApplySplitMax && n_tasks * s < kApplySplitWaves) s *= 2;
+  return s;
 }
 
 void launch_apply(int W, int mode, bool fill, const ApplyArgs& a, hipStream_t s) {

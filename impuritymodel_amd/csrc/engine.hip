@@ -383,12 +383,24 @@ __global__ void layer_grow_kernel(const int32_t* pool_chain, int64_t P0, int64_t
   if (i == n - 1 || pool_chain[P0 + i + 1] != c) chain_size[c] += i - seg_start[c] + 1;
 }
 
-__global__ void record_cols_kernel(const int64_t* offsets, const int32_t* counts, int64_t n, int64_t base,
+// First entry of source i: its first part's offset (total past the last source).
+__device__ __forceinline__ int64_t source_offset(const int64_t* offsets, int split, int64_t n, int64_t total,
+                                                 int64_t i) {
+  return i < n ? offsets[i * split] : total;
+}
+
+__global__ void record_cols_kernel(const int64_t* offsets, int split, int64_t n, int64_t total, int64_t base,
                                    int64_t* pool_coloff, int32_t* pool_colcnt, int64_t P0) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  pool_coloff[P0 + i] = base + offsets[i];
-  pool_colcnt[P0 + i] = counts[i];
+  const int64_t a = source_offset(offsets, split, n, total, i);
+  pool_coloff[P0 + i] = base + a;
+  pool_colcnt[P0 + i] = (int32_t)(source_offset(offsets, split, n, total, i + 1) - a);
+}
+
+__global__ void source_rowptr_kernel(const int64_t* offsets, int split, int64_t n, int64_t total, int64_t* rowptr) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n) rowptr[i] = source_offset(offsets, split, n, total, i);
 }
 
 __global__ void row_order_kernel(const int32_t* pool_chain, const int32_t* pool_local, const int64_t* row_base,
@@ -526,22 +538,24 @@ static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double we
   a.n_tasks = nt;
   a.src_keys = b.pool_keys.as<uint64_t>();
   a.weight_min = weight_min;
-  sc.counts.reserve(n * sizeof(int32_t));
+  a.split = apply_split(nt);
+  const int64_t nc = n * a.split;  // counts: one per (source, part)
+  sc.counts.reserve(nc * sizeof(int32_t));
   // the wave tasks carry absolute source ids; counts/offsets are indexed the
   // same way through a shifted base pointer
-  a.counts = sc.counts.as<int32_t>() - f0;
+  a.counts = sc.counts.as<int32_t>() - f0 * a.split;
   a.hash = hash_view(b);
   a.pool_local = b.pool_local.as<int32_t>();
   launch_apply(b.W, mode, false, a, stream());
-  sc.offsets.reserve((n + 1) * sizeof(int64_t));
-  int64_t E = scan_counts(sc.counts.as<int32_t>(), n, sc.offsets.as<int64_t>(), stream());
-  a.offsets = sc.offsets.as<int64_t>() - f0;
+  sc.offsets.reserve((nc + 1) * sizeof(int64_t));
+  int64_t E = scan_counts(sc.counts.as<int32_t>(), nc, sc.offsets.as<int64_t>(), stream());
+  a.offsets = sc.offsets.as<int64_t>() - f0 * a.split;
   if (mode == MODE_EXPAND) {
     int64_t base = b.E;
     b.col_keys.grow_keep((base + E) * b.W * 8, base * b.W * 8, stream());
     b.col_val.grow_keep((base + E) * 16, base * 16, stream());
     hipLaunchKernelGGL(record_cols_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream(), sc.offsets.as<int64_t>(),
-                       sc.counts.as<int32_t>(), n, base, b.pool_coloff.as<int64_t>(), b.pool_colcnt.as<int32_t>(), f0);
+                       a.split, n, E, base, b.pool_coloff.as<int64_t>(), b.pool_colcnt.as<int32_t>(), f0);
     ensure_hash(b, b.P + E);
     a.hash = hash_view(b);
     sc.cand_keys.reserve(std::max<int64_t>(E, 1) * b.W * 8);
@@ -554,7 +568,6 @@ static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double we
     a.out_val = b.col_val.as<double2>() + base;
     sc.col_chain.reserve(std::max<int64_t>(E, 1) * 4);
     a.out_chain = sc.col_chain.as<int32_t>();
-    a.offsets = sc.offsets.as<int64_t>() - f0;
     a.cand = CandView{sc.cand_keys.as<uint64_t>(), sc.cand_chain.as<int32_t>(), sc.cand_slot.as<int32_t>(),
                       sc.cand_cnt.as<int32_t>(),   sc.alive.as<int32_t>(),      sc.cand_cnt.as<int32_t>() + 1,
                       (int32_t)std::min<int64_t>(E, INT32_MAX)};
@@ -570,9 +583,9 @@ static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double we
   } else {
     // fixed basis: write the CSR directly (rows are pool ids = local ids)
     b.rowptr.reserve((n + 1) * sizeof(int64_t));
-    HIP_CHECK(hipMemcpyAsync(b.rowptr.p, sc.offsets.p, n * sizeof(int64_t), hipMemcpyDeviceToDevice, stream()));
-    HIP_CHECK(hipMemcpyAsync(b.rowptr.as<int64_t>() + n, &E, sizeof(int64_t), hipMemcpyHostToDevice, stream()));
-    stream_sync(stream());
+    hipLaunchKernelGGL(source_rowptr_kernel, dim3(blocks_for(n + 1, 256)), dim3(256), 0, stream(),
+                       sc.offsets.as<int64_t>(), a.split, n, E, b.rowptr.as<int64_t>());
+    HIP_CHECK(hipGetLastError());
     b.col.reserve(std::max<int64_t>(E, 1) * 4);
     b.val.reserve(std::max<int64_t>(E, 1) * 16);
     a.out_col = b.col.as<int32_t>();

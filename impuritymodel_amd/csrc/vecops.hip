@@ -240,11 +240,13 @@ void vector_apply(OpsView ops, int W, const std::vector<int64_t>& src_off, const
   a.src_amps = sc.samps.as<double2>();
   a.src_pos = sc.spos.as<int32_t>();
   a.weight_min = weight_min;
-  sc.counts.reserve(NS * 4);
+  a.split = apply_split(a.n_tasks);
+  const int64_t NC = NS * a.split;  // counts: one per (source, part)
+  sc.counts.reserve(NC * 4);
   a.counts = sc.counts.as<int32_t>();
   launch_apply(W, MODE_VECTOR, false, a, s);
-  sc.offs.reserve((NS + 1) * 8);
-  const int64_t E = scan_counts(sc.counts.as<int32_t>(), NS, sc.offs.as<int64_t>(), s);
+  sc.offs.reserve((NC + 1) * 8);
+  const int64_t E = scan_counts(sc.counts.as<int32_t>(), NC, sc.offs.as<int64_t>(), s);
   if (E == 0) {
     out_keys.reserve(8);
     out_amps.reserve(16);
