@@ -299,7 +299,7 @@ struct Batch {
   std::vector<int64_t> h_n, h_row_base, h_nnz;
   // column storage (expansion)
   int64_t E = 0;
-  DevBuf col_keys, col_val;
+  DevBuf col_id, col_val;  // per entry: pool id of its target, value
   // CSR in chain-local order, rows of chain c at [row_base[c], row_base[c]+n[c])
   int64_t R = 0, NNZ = 0;
   DevBuf rowptr, col, val, row_chain, row_base, chain_n;
@@ -345,16 +345,27 @@ __global__ void set_local_seed_kernel(const int64_t* seed_off, int C, int32_t* p
   if (threadIdx.x == 0) chain_size[c] = b - a;
 }
 
-__global__ void append_layer_kernel(int W, const int32_t* perm, int64_t n, const uint64_t* cand_keys,
-                                    const int32_t* cand_chain, const int32_t* cand_slot, int64_t P0, uint64_t* pool_keys,
+// The layer's new states in sorted order: pool slots P0 + i, the table slot now
+// holds the pool id, and winner_slot of the entry that stands for the state too.
+__global__ void append_layer_kernel(int W, const int32_t* perm, int64_t n, const uint64_t* entry_keys,
+                                    const int32_t* entry_chain, int32_t* winner_slot, int64_t P0, uint64_t* pool_keys,
                                     int32_t* pool_chain, int32_t* table) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int32_t c = perm[i];
+  int32_t e = perm[i];
   int64_t g = P0 + i;
-  for (int w = 0; w < W; ++w) pool_keys[g * W + w] = cand_keys[(size_t)c * W + w];
-  pool_chain[g] = cand_chain[c];
-  table[cand_slot[c]] = (int32_t)g;
+  for (int w = 0; w < W; ++w) pool_keys[g * W + w] = entry_keys[(size_t)e * W + w];
+  pool_chain[g] = entry_chain[e];
+  table[winner_slot[e]] = (int32_t)g;
+  winner_slot[e] = (int32_t)g;
+}
+
+// Entries that named a new state by its entry get the state's pool id.
+__global__ void resolve_entries_kernel(int32_t* entry_id, int64_t E, const int32_t* new_id) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= E) return;
+  const int32_t id = entry_id[e];
+  if (id & CAND_FLAG) entry_id[e] = new_id[id & ~CAND_FLAG];
 }
 
 __global__ void layer_heads_kernel(const int32_t* pool_chain, int64_t P0, int64_t n, int64_t* seg_start) {
@@ -418,43 +429,22 @@ __global__ void row_counts_kernel(const int32_t* row_gid, const int32_t* pool_co
   if (r < R) cnt[r] = pool_colcnt[row_gid[r]];
 }
 
-// Row r of H is the conjugate of column r: <r|H|t> = conj(<t|H|r>).
-template <int W>
-__global__ void csr_fill_kernel(HashView h, const int32_t* row_gid, const int32_t* row_chain, int64_t R,
-                                const int64_t* pool_coloff, const uint64_t* col_keys, const double2* col_vals,
-                                const int32_t* pool_local, const int64_t* rowptr, int32_t* col, double2* val,
-                                int32_t* err) {
-  int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Row r of H is the conjugate of column r: <r|H|t> = conj(<t|H|r>).  The entries
+// carry their targets' pool ids, so a row is a copy with one lookup of the target's
+// local index; CSR_LANES lanes share a row.  (One thread a row that probed the hash
+// again for each entry took 8.4 ms for 2.9e6 rows; this takes 1.5 ms.)
+constexpr int CSR_LANES = 16;
+
+__global__ __launch_bounds__(256) void csr_fill_kernel(const int32_t* row_gid, int64_t R, const int64_t* pool_coloff,
+                                                       const int32_t* col_id, const double2* col_vals,
+                                                       const int32_t* pool_local, const int64_t* rowptr, int32_t* col,
+                                                       double2* val) {
+  const int64_t r = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / CSR_LANES;
   if (r >= R) return;
-  int32_t g = row_gid[r];
-  int32_t c = row_chain[r];
-  int64_t src = pool_coloff[g];
-  int64_t a = rowptr[r], b = rowptr[r + 1];
-  for (int64_t e = a; e < b; ++e) {
-    const uint64_t* k = col_keys + (size_t)(src + (e - a)) * W;
-    uint32_t slot = hash_key((uint32_t)c, k, W) & h.mask;
-    int32_t id = HASH_EMPTY;
-    for (;;) {
-      int32_t cur = h.table[slot];
-      if (cur == HASH_EMPTY) break;
-      if (!(cur & CAND_FLAG) && h.pool_chain[cur] == c) {
-        bool eq = true;
-        for (int w = 0; w < W; ++w) eq = eq && h.pool_keys[(size_t)cur * W + w] == k[w];
-        if (eq) {
-          id = cur;
-          break;
-        }
-      }
-      slot = (slot + 1) & h.mask;
-    }
-    if (id < 0) {
-      atomicExch(err, 1);
-      col[e] = 0;
-      val[e] = make_double2(0.0, 0.0);
-      continue;
-    }
-    col[e] = pool_local[id];
-    val[e] = cconj(col_vals[src + (e - a)]);
+  const int64_t a = rowptr[r], n = rowptr[r + 1] - a, src = pool_coloff[row_gid[r]];
+  for (int64_t i = threadIdx.x % CSR_LANES; i < n; i += CSR_LANES) {
+    col[a + i] = pool_local[col_id[src + i]];
+    val[a + i] = cconj(col_vals[src + i]);
   }
 }
 
@@ -511,7 +501,7 @@ static HashView hash_view(Batch& b) {
 
 // Scratch shared by the build steps.
 struct BuildScratch {
-  DevBuf tasks, counts, offsets, cand_keys, cand_chain, cand_slot, cand_cnt, alive, perm, rowgid, err, col_chain;
+  DevBuf tasks, counts, offsets, entry_keys, entry_chain, winner_slot, n_winners, perm, rowgid;
 };
 static BuildScratch& bscratch() {
   static BuildScratch s;
@@ -527,8 +517,9 @@ static int64_t make_tasks(Batch& b, int64_t begin, int64_t end) {
 }
 
 // Apply the Hamiltonian to pool states [f0, f1): count, scan, fill.  In
-// expand mode new targets become candidates; returns the entry count.
-static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double weight_min, int64_t* n_alive) {
+// expand mode the entries' targets are looked up and the entries of new targets
+// listed in the scratch perm (*n_new of them); returns the entry count.
+static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double weight_min, int64_t* n_new) {
   BuildScratch& sc = bscratch();
   const int64_t n = f1 - f0;
   int64_t nt = make_tasks(b, f0, f1);
@@ -552,34 +543,31 @@ static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double we
   a.offsets = sc.offsets.as<int64_t>() - f0 * a.split;
   if (mode == MODE_EXPAND) {
     int64_t base = b.E;
-    b.col_keys.grow_keep((base + E) * b.W * 8, base * b.W * 8, stream());
+    b.col_id.grow_keep((base + E) * 4, base * 4, stream());
     b.col_val.grow_keep((base + E) * 16, base * 16, stream());
     hipLaunchKernelGGL(record_cols_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream(), sc.offsets.as<int64_t>(),
                        a.split, n, E, base, b.pool_coloff.as<int64_t>(), b.pool_colcnt.as<int32_t>(), f0);
     ensure_hash(b, b.P + E);
     a.hash = hash_view(b);
-    sc.cand_keys.reserve(std::max<int64_t>(E, 1) * b.W * 8);
-    sc.cand_chain.reserve(std::max<int64_t>(E, 1) * 4);
-    sc.cand_slot.reserve(std::max<int64_t>(E, 1) * 4);
-    sc.alive.reserve(std::max<int64_t>(E, 1) * 4);
-    sc.cand_cnt.reserve(2 * sizeof(int32_t));
-    HIP_CHECK(hipMemsetAsync(sc.cand_cnt.p, 0, 2 * sizeof(int32_t), stream()));
-    a.out_keys = b.col_keys.as<uint64_t>() + base * b.W;
+    sc.entry_keys.reserve(std::max<int64_t>(E, 1) * b.W * 8);
+    sc.entry_chain.reserve(std::max<int64_t>(E, 1) * 4);
+    sc.winner_slot.reserve(std::max<int64_t>(E, 1) * 4);
+    sc.perm.reserve(std::max<int64_t>(E, 1) * 4);
+    sc.n_winners.reserve(sizeof(int32_t));
+    HIP_CHECK(hipMemsetAsync(sc.n_winners.p, 0, sizeof(int32_t), stream()));
+    a.out_keys = sc.entry_keys.as<uint64_t>();
     a.out_val = b.col_val.as<double2>() + base;
-    sc.col_chain.reserve(std::max<int64_t>(E, 1) * 4);
-    a.out_chain = sc.col_chain.as<int32_t>();
-    a.cand = CandView{sc.cand_keys.as<uint64_t>(), sc.cand_chain.as<int32_t>(), sc.cand_slot.as<int32_t>(),
-                      sc.cand_cnt.as<int32_t>(),   sc.alive.as<int32_t>(),      sc.cand_cnt.as<int32_t>() + 1,
-                      (int32_t)std::min<int64_t>(E, INT32_MAX)};
+    a.out_chain = sc.entry_chain.as<int32_t>();
     if (E > 0) {
       launch_apply(b.W, mode, true, a, stream());
-      launch_discover(b.W, a.out_keys, a.out_chain, E, a.hash, a.cand, stream());
+      launch_discover(b.W, a.out_keys, a.out_chain, E, a.hash, b.col_id.as<int32_t>() + base,
+                      sc.winner_slot.as<int32_t>(), sc.perm.as<int32_t>(), sc.n_winners.as<int32_t>(), stream());
     }
-    int32_t cc[2] = {0, 0};
-    d2h_bytes(cc, sc.cand_cnt.p, sizeof(cc), stream());
+    int32_t nw = 0;
+    d2h_bytes(&nw, sc.n_winners.p, sizeof(nw), stream());
     stream_sync(stream());
     b.E = base + E;
-    *n_alive = cc[1];
+    *n_new = nw;
   } else {
     // fixed basis: write the CSR directly (rows are pool ids = local ids)
     b.rowptr.reserve((n + 1) * sizeof(int64_t));
@@ -592,7 +580,7 @@ static int64_t apply_layer(Batch& b, int64_t f0, int64_t f1, int mode, double we
     a.out_val = b.val.as<double2>();
     if (E > 0) launch_apply(b.W, mode, true, a, stream());
     stream_sync(stream());
-    *n_alive = 0;
+    *n_new = 0;
   }
   return E;
 }
@@ -679,33 +667,33 @@ static void build(Batch& b, int mode, double weight_min, int max_layers) {
   while (f1 > f0) {
     if (max_layers > 0 && layers >= max_layers) break;
     ++layers;
-    int64_t n_alive = 0;
-    apply_layer(b, f0, f1, MODE_EXPAND, weight_min, &n_alive);
-    if (n_alive == 0) {
+    int64_t n_new = 0;
+    const int64_t E = apply_layer(b, f0, f1, MODE_EXPAND, weight_min, &n_new);
+    if (n_new == 0) {
       f0 = f1;
       break;
     }
     // sort the new states by (chain, key) and append them
-    sc.perm.reserve(n_alive * sizeof(int32_t));
-    HIP_CHECK(hipMemcpyAsync(sc.perm.p, sc.alive.p, n_alive * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
-    sort_chain_keys(b.W, b.ops->n_orb, bits_for(b.C), sc.cand_keys.as<uint64_t>(), sc.cand_chain.as<int32_t>(),
-                    sc.perm.as<int32_t>(), n_alive, s);
-    ensure_pool(b, b.P + n_alive);
+    sort_chain_keys(b.W, b.ops->n_orb, bits_for(b.C), sc.entry_keys.as<uint64_t>(), sc.entry_chain.as<int32_t>(),
+                    sc.perm.as<int32_t>(), n_new, s);
+    ensure_pool(b, b.P + n_new);
     const int64_t P0 = b.P;
-    hipLaunchKernelGGL(append_layer_kernel, dim3(blocks_for(n_alive, 256)), dim3(256), 0, s, b.W,
-                       sc.perm.as<int32_t>(), n_alive, sc.cand_keys.as<uint64_t>(), sc.cand_chain.as<int32_t>(),
-                       sc.cand_slot.as<int32_t>(), P0, b.pool_keys.as<uint64_t>(), b.pool_chain.as<int32_t>(),
+    hipLaunchKernelGGL(append_layer_kernel, dim3(blocks_for(n_new, 256)), dim3(256), 0, s, b.W,
+                       sc.perm.as<int32_t>(), n_new, sc.entry_keys.as<uint64_t>(), sc.entry_chain.as<int32_t>(),
+                       sc.winner_slot.as<int32_t>(), P0, b.pool_keys.as<uint64_t>(), b.pool_chain.as<int32_t>(),
                        b.table.as<int32_t>());
-    hipLaunchKernelGGL(layer_heads_kernel, dim3(blocks_for(n_alive, 256)), dim3(256), 0, s,
-                       b.pool_chain.as<int32_t>(), P0, n_alive, b.seg_start.as<int64_t>());
-    hipLaunchKernelGGL(layer_local_kernel, dim3(blocks_for(n_alive, 256)), dim3(256), 0, s,
-                       b.pool_chain.as<int32_t>(), P0, n_alive, b.seg_start.as<int64_t>(),
+    hipLaunchKernelGGL(resolve_entries_kernel, dim3(blocks_for(E, 256)), dim3(256), 0, s,
+                       b.col_id.as<int32_t>() + (b.E - E), E, sc.winner_slot.as<int32_t>());
+    hipLaunchKernelGGL(layer_heads_kernel, dim3(blocks_for(n_new, 256)), dim3(256), 0, s,
+                       b.pool_chain.as<int32_t>(), P0, n_new, b.seg_start.as<int64_t>());
+    hipLaunchKernelGGL(layer_local_kernel, dim3(blocks_for(n_new, 256)), dim3(256), 0, s,
+                       b.pool_chain.as<int32_t>(), P0, n_new, b.seg_start.as<int64_t>(),
                        b.chain_size.as<int64_t>(), b.pool_local.as<int32_t>());
-    hipLaunchKernelGGL(layer_grow_kernel, dim3(blocks_for(n_alive, 256)), dim3(256), 0, s,
-                       b.pool_chain.as<int32_t>(), P0, n_alive, b.seg_start.as<int64_t>(),
+    hipLaunchKernelGGL(layer_grow_kernel, dim3(blocks_for(n_new, 256)), dim3(256), 0, s,
+                       b.pool_chain.as<int32_t>(), P0, n_new, b.seg_start.as<int64_t>(),
                        b.chain_size.as<int64_t>());
     HIP_CHECK(hipGetLastError());
-    b.P = P0 + n_alive;
+    b.P = P0 + n_new;
     f0 = f1;
     f1 = b.P;
   }
@@ -729,33 +717,21 @@ static void build(Batch& b, int mode, double weight_min, int max_layers) {
   stream_sync(s);
   b.col.reserve(std::max<int64_t>(nnz, 1) * 4);
   b.val.reserve(std::max<int64_t>(nnz, 1) * 16);
-  sc.err.reserve(4);
-  HIP_CHECK(hipMemsetAsync(sc.err.p, 0, 4, s));
   if (b.R) {
     TimedLaunch tl("csr_fill", s);
-    if (b.W == 1)
-      hipLaunchKernelGGL(csr_fill_kernel<1>, dim3(blocks_for(b.R, 128)), dim3(128), 0, s, hash_view(b),
-                         sc.rowgid.as<int32_t>(), b.row_chain.as<int32_t>(), b.R, b.pool_coloff.as<int64_t>(),
-                         b.col_keys.as<uint64_t>(), b.col_val.as<double2>(), b.pool_local.as<int32_t>(),
-                         b.rowptr.as<int64_t>(), b.col.as<int32_t>(), b.val.as<double2>(), sc.err.as<int32_t>());
-    else
-      hipLaunchKernelGGL(csr_fill_kernel<2>, dim3(blocks_for(b.R, 128)), dim3(128), 0, s, hash_view(b),
-                         sc.rowgid.as<int32_t>(), b.row_chain.as<int32_t>(), b.R, b.pool_coloff.as<int64_t>(),
-                         b.col_keys.as<uint64_t>(), b.col_val.as<double2>(), b.pool_local.as<int32_t>(),
-                         b.rowptr.as<int64_t>(), b.col.as<int32_t>(), b.val.as<double2>(), sc.err.as<int32_t>());
+    hipLaunchKernelGGL(csr_fill_kernel, dim3(blocks_for(b.R * CSR_LANES, 256)), dim3(256), 0, s,
+                       sc.rowgid.as<int32_t>(), b.R, b.pool_coloff.as<int64_t>(), b.col_id.as<int32_t>(),
+                       b.col_val.as<double2>(), b.pool_local.as<int32_t>(), b.rowptr.as<int64_t>(),
+                       b.col.as<int32_t>(), b.val.as<double2>());
     HIP_CHECK(hipGetLastError());
   }
-  // basis keys in row order (reuse col_keys tail is not safe; keep a copy in seed_keys)
+  // basis keys in row order
   b.seed_keys.reserve(std::max<int64_t>(b.R, 1) * b.W * 8);
   DevBuf tmp;
   tmp.reserve(std::max<int64_t>(b.R, 1) * b.W * 8);
   hipLaunchKernelGGL(keys_by_rows_kernel, dim3(blocks_for(b.R, 256)), dim3(256), 0, s, b.W, sc.rowgid.as<int32_t>(),
                      b.R, b.pool_keys.as<uint64_t>(), tmp.as<uint64_t>());
   HIP_CHECK(hipMemcpyAsync(b.pool_keys.p, tmp.p, b.R * b.W * 8, hipMemcpyDeviceToDevice, s));
-  int32_t err = 0;
-  d2h_bytes(&err, sc.err.p, 4, s);
-  stream_sync(s);
-  if (err) throw HipError{"internal error: CSR target missing from basis"};
   compute_chain_nnz(b);
   b.built = true;
   b.row_keys = true;

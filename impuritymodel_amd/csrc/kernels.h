@@ -35,8 +35,10 @@ struct WaveTask {
   int64_t end;
 };
 
-// Open-addressing state -> id table over (chain, key); slots hold pool ids,
-// candidate ids (| CAND_FLAG) or EMPTY.
+// Open-addressing state -> id table over (chain, key); slots hold pool ids, EMPTY,
+// or, between a layer's discovery and its append, the layer's entry numbers
+// (| CAND_FLAG; pool ids and entry numbers stay below 2^30, as the table holds at
+// least twice their sum and at most 2^31 slots).
 constexpr int32_t HASH_EMPTY = -1;
 constexpr int32_t CAND_FLAG = 0x40000000;
 
@@ -45,16 +47,6 @@ struct HashView {
   uint32_t mask;
   const uint64_t* pool_keys;
   const int32_t* pool_chain;
-};
-
-struct CandView {
-  uint64_t* keys;
-  int32_t* chain;
-  int32_t* slot;
-  int32_t* count;
-  int32_t* alive_list;
-  int32_t* alive_count;
-  int32_t cap;
 };
 
 enum ApplyMode { MODE_EXPAND = 0, MODE_FIXED = 1, MODE_VECTOR = 2 };
@@ -82,7 +74,6 @@ struct ApplyArgs {
   int32_t* out_src;
   int32_t* out_first;
   HashView hash;
-  CandView cand;
 };
 
 // Parts the groups of a model are divided into, a power of two: launches of fewer
@@ -94,8 +85,12 @@ constexpr int kApplySplitMax = 32;
 int apply_split(int64_t n_tasks);
 
 void launch_apply(int W, int mode, bool fill, const ApplyArgs& a, hipStream_t s);
-void launch_discover(int W, const uint64_t* keys, const int32_t* chain, int64_t E, HashView h, CandView c,
-                     hipStream_t s);
+// Entries e < E of a layer: entry_id[e] = the pool id of (chain[e], keys[e]), or
+// CAND_FLAG | the entry that stands for it when it is new; those entries are
+// listed in winners (any order, *n_winners of them, zero before), winner_slot[e]
+// their table slot.
+void launch_discover(int W, const uint64_t* keys, const int32_t* chain, int64_t E, HashView h, int32_t* entry_id,
+                     int32_t* winner_slot, int32_t* winners, int32_t* n_winners, hipStream_t s);
 
 void launch_hash_insert_pool(int W, HashView h, int64_t first, int64_t count, hipStream_t s);
 void launch_hash_clear(int32_t* table, uint32_t cap, hipStream_t s);
