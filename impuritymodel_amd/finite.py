@@ -22,7 +22,7 @@ import numpy as np
 import scipy.sparse
 
 from . import opcompile
-from .engine import Batch, Ops, vec_apply, vec_from_host
+from .engine import Batch, Ops, Vec, vec_apply, vec_from_host
 from .operators import (  # noqa: F401  (reference names)
     addOps,
     assert_hermitian,
@@ -92,28 +92,37 @@ def applyOp(n_spin_orbitals, op, psi, slaterWeightMin=1e-12, restrictions=None, 
         k, a, _ = out.get()
         return dict(zip(opcompile.words_to_bytes(k, n), a.tolist()))
     new_states = [s for s in psi if s not in opResult]
-    per_state = {}
-    if new_states:
-        words = _words(new_states, n)
-        src = vec_from_host(W, [words[i:i + 1] for i in range(len(new_states))],
-                            [np.ones(1, complex)] * len(new_states))
-        out = vec_apply(ops, src, np.arange(len(new_states)), np.zeros(len(new_states), np.int32), 0.0)
-        k, a, _ = out.get()
-        off = out.offsets
-        kb = opcompile.words_to_bytes(k, n)
-        for i, s in enumerate(new_states):
-            per_state[s] = list(zip(kb[off[i]:off[i + 1]], a[off[i]:off[i + 1]].tolist()))
+    return _memo_sum(psi, _state_results(n, ops, 1, new_states)[0], slaterWeightMin, opResult)
+
+
+def _state_results(n, ops, n_models, states):
+    """Per model of ``ops`` a dict {state: [(target, value), ...]}, the targets in
+    the operator's order and unpruned, from one batched application."""
+    if not states:
+        return [{} for _ in range(n_models)]
+    ns = len(states)
+    src = Vec(ops.W, keys=_words(states, n), amps=np.ones(ns, complex), offsets=np.arange(ns + 1, dtype=np.int64))
+    out = vec_apply(ops, src, np.tile(np.arange(ns), n_models), np.repeat(np.arange(n_models), ns), 0.0)
+    k, a, _ = out.get()
+    off = out.offsets.tolist()
+    entries = list(zip(opcompile.words_to_bytes(k, n), a.tolist()))
+    return [{s: entries[off[m * ns + i]:off[m * ns + i + 1]] for i, s in enumerate(states)} for m in range(n_models)]
+
+
+def _memo_sum(psi, per_state, slaterWeightMin, opResult):
+    """op|psi> from the memo ``opResult`` and, for states it does not hold, the
+    results ``per_state``, which it stores (finite.py:1413-1504)."""
     psi_new = {}
     for state, amp in psi.items():
-        if state in per_state:
+        if state in opResult:
+            for t, v in opResult[state].items():
+                psi_new[t] = psi_new[t] + v * amp if t in psi_new else v * amp
+        else:
             memo = {}
             for t, v in per_state[state]:
                 psi_new[t] = psi_new[t] + amp * v if t in psi_new else amp * v
                 memo[t] = v
             opResult[state] = {t: v for t, v in memo.items() if abs(v) ** 2 >= slaterWeightMin}
-        else:
-            for t, v in opResult[state].items():
-                psi_new[t] = psi_new[t] + v * amp if t in psi_new else v * amp
     return {s: a for s, a in psi_new.items() if abs(a) ** 2 >= slaterWeightMin}
 
 

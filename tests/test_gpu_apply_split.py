@@ -92,3 +92,28 @@ def test_build_split(gpu, n_bath, fixed):
         assert np.array_equal(col.reshape(copies, nnz), np.tile(ref[1], (copies, 1)))
         assert np.array_equal(val.reshape(copies, nnz), np.tile(ref[2], (copies, 1)))
         assert np.array_equal(bt.basis_words(), np.tile(ref[3], (copies, 1)))
+
+
+@pytest.mark.parametrize("vectors", [1, 100, 1 << 20])
+@pytest.mark.parametrize("n_op,n_psi,size", [(1, 1, 1), (7, 3, 40), (3, 2, 0)])
+def test_batched_memo_equals_one_by_one(gpu, monkeypatch, vectors, n_op, n_psi, size):
+    """Transition states of all operators from one application against applyOp with a
+    memo per operator, one state after the other: the same bits in the same order."""
+    from impuritymodel_amd import finite, opcompile, spectra
+
+    n = 20
+    rng = np.random.default_rng(size)
+    t_ops = [_operator(n, 5 + 3 * i, i) for i in range(n_op)]
+    pool = [opcompile.words_to_bytes(np.array([[int(x) << (64 - n)]], np.uint64), n)[0]
+            for x in rng.choice(1 << n, 60, replace=False)]
+    psis = [{pool[i]: complex(*rng.normal(size=2)) for i in rng.permutation(60)[:size]} for _ in range(n_psi)]
+    restr = {frozenset(range(8)): (1, 6)}
+    ref = []
+    for op in t_ops:
+        memo = {}
+        ref += [finite.applyOp(n, op, psi, 0.5, restr, memo) for psi in psis]
+    monkeypatch.setattr(spectra, "_MEMO_VECTORS", vectors)
+    keys, amps = spectra._transition_states_memo(n, t_ops, psis, 0.5, restr)
+    assert len(keys) == len(amps) == len(ref)
+    for k, a, r in zip(keys, amps, ref):
+        assert opcompile.words_to_bytes(k, n) == list(r) and a.tolist() == list(r.values())
