@@ -70,19 +70,41 @@ __device__ __forceinline__ double lane_f64(double v, int i) {
   return __longlong_as_double((long long)lane_u64((uint64_t)__double_as_longlong(v), i));
 }
 
-// 64 terms (one per lane) and 64 groups (one per lane) of the tables.
+// 64 terms, one per lane.  A state that matches has val on the care bits, so the
+// part of its sign that those bits decide goes into the coefficient once, here
+// (a negation is exact), and sgn keeps the other bits; terms without such bits, or
+// without an imaginary part, skip that work by a wave-uniform bit test.
 template <int W>
 struct TermChunk {
-  uint64_t m[3 * W];
+  uint64_t care[W], val[W], sgn[W];
   double2 c;
   uint32_t meta;
   __device__ __forceinline__ void load(const OpsView& o, int t, int t_end) {
     if (t < t_end) {
 #pragma unroll
-      for (int w = 0; w < 3 * W; ++w) m[w] = o.term_masks[(size_t)t * 3 * W + w];
+      for (int w = 0; w < W; ++w) {
+        const uint64_t* m = o.term_masks + (size_t)t * 3 * W + w;
+        care[w] = m[0];
+        val[w] = m[W];
+        sgn[w] = m[2 * W];
+      }
       c = o.term_coef[t];
       meta = o.term_meta[t];
     }
+  }
+  // terms with sign bits left, terms with an imaginary part
+  __device__ __forceinline__ void fold(uint64_t& has_sign, uint64_t& has_imag) {
+    uint32_t par = meta & 1u;
+    uint64_t left = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      par ^= (uint32_t)__popcll(val[w] & sgn[w]) & 1u;
+      sgn[w] &= ~care[w];
+      left |= sgn[w];
+    }
+    if (par) c = make_double2(-c.x, -c.y);
+    has_sign = __ballot(left != 0);
+    has_imag = __ballot(!(c.y == 0.0));
   }
 };
 
@@ -91,11 +113,12 @@ struct TermChunk {
 // terms, and counts and offsets hold one value per (source, part), so the
 // entries of a source stay in group order whatever the split is.
 //
-// What bounds it: instruction issue of the walk over the terms, about 30 vector
-// instructions a term with a match and 10 without.  Measured on 1100-term models,
-// one launch: a few hundred sources 130 us with the terms in LDS and one wave per
-// task, 45 us so (the number operators are one group of hundreds of matching
-// terms, which stays with one wave); 3e6 sources of two words 1.6 to 1.1 ms.
+// What bounds it: instruction issue of the walk over the terms, 65 to 200 cycles a
+// term.  Measured on 1000-term models, one launch: a few hundred sources 130 us with
+// the terms in LDS and one wave per task, 45 us from registers with the groups
+// divided, 24 us with the signs folded and the number operators' branches gone
+// (they are one group of 340 matching terms, which stays with one wave); up to 3e6
+// sources of two words 1.6, 1.1 and 0.95 ms.
 template <int W, int MODE, bool FILL>
 __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
   __shared__ uint64_t l_rmask[4][RESTR_LDS * W];
@@ -155,8 +178,10 @@ __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
 
   TermChunk<W> cur{}, next{};
   int tc0 = t;  // first term of the chunk in registers
+  uint64_t has_sign, has_imag;
   cur.load(o, tc0 + lane, t_end);
   next.load(o, tc0 + 64 + lane, t_end);
+  cur.fold(has_sign, has_imag);
   int gc0 = g0;  // first group in registers
   int32_t gend = 0;
   uint64_t gflip[W] = {};
@@ -180,38 +205,52 @@ __global__ __launch_bounds__(256) void apply_kernel(ApplyArgs a) {
     int first = 0;
     // one matching term: add its signed value (in term order)
     auto take = [&](int i) {
-      const uint32_t meta = __builtin_amdgcn_readlane(cur.meta, i);
-      uint32_t par = meta & 1u;
+      double cx = lane_f64(cur.c.x, i), cy = 0.0;
+      if (has_imag >> i & 1) cy = lane_f64(cur.c.y, i);
+      if (has_sign >> i & 1) {
+        uint32_t par = 0;
 #pragma unroll
-      for (int w = 0; w < W; ++w) par ^= (uint32_t)__popcll(s[w] & lane_u64(cur.m[2 * W + w], i)) & 1u;
-      const double cx = lane_f64(cur.c.x, i), cy = lane_f64(cur.c.y, i);
-      if (par) {
-        acc.x -= cx;
-        acc.y -= cy;
-      } else {
-        acc.x += cx;
-        acc.y += cy;
+        for (int w = 0; w < W; ++w) par ^= (uint32_t)__popcll(s[w] & lane_u64(cur.sgn[w], i)) & 1u;
+        cx = par ? -cx : cx;
+        cy = par ? -cy : cy;
       }
-      if (!any) first = (int)(meta >> 1);
+      acc.x += cx;
+      if (has_imag >> i & 1) acc.y += cy;
+      if (MODE == MODE_VECTOR && !any) first = (int)(__builtin_amdgcn_readlane(cur.meta, i) >> 1);
       any = true;
     };
     auto matches = [&](int i) {
-      uint64_t diff = 0;
+      bool ok = true;
 #pragma unroll
-      for (int w = 0; w < W; ++w) diff |= (s[w] & lane_u64(cur.m[w], i)) ^ lane_u64(cur.m[W + w], i);
-      return diff == 0;
+      for (int w = 0; w < W; ++w) ok = ok & ((s[w] & lane_u64(cur.care[w], i)) == lane_u64(cur.val[w], i));
+      return ok;
     };
     while (t < te) {
       if (t - tc0 == 64) {
         tc0 = t;
         cur = next;
         next.load(o, tc0 + 64 + lane, t_end);
+        cur.fold(has_sign, has_imag);
       }
       const int iend = te - tc0 < 64 ? te - tc0 : 64;
       int i = t - tc0;
-      // four mask tests at once, the matches taken in term order
+      // Four mask tests at once, the matches taken in term order.  Where the four
+      // are real and their signs are decided (number operators), adding 0 in the
+      // lanes without a match takes the place of four branches; the sum is never
+      // -0, so that adds nothing.
       for (; i + 4 <= iend; i += 4) {
         const bool k0 = matches(i), k1 = matches(i + 1), k2 = matches(i + 2), k3 = matches(i + 3);
+        if (__ballot(k0 | k1 | k2 | k3) == 0) continue;
+        if (MODE != MODE_VECTOR && ((has_sign | has_imag) >> i & 15) == 0) {
+          const double c0 = lane_f64(cur.c.x, i), c1 = lane_f64(cur.c.x, i + 1);
+          const double c2 = lane_f64(cur.c.x, i + 2), c3 = lane_f64(cur.c.x, i + 3);
+          acc.x += k0 ? c0 : 0.0;
+          acc.x += k1 ? c1 : 0.0;
+          acc.x += k2 ? c2 : 0.0;
+          acc.x += k3 ? c3 : 0.0;
+          any = any | k0 | k1 | k2 | k3;
+          continue;
+        }
         if (k0) take(i);
         if (k1) take(i + 1);
         if (k2) take(i + 2);

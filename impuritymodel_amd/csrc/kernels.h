@@ -78,7 +78,7 @@ struct ApplyArgs {
 
 // Parts the groups of a model are divided into, a power of two: launches of fewer
 // than kApplySplitWaves wave tasks (two waves per SIMD) spread each task's terms
-// over more waves.  A launch of 1 to 20 tasks takes 130 us undivided and 45 us in
+// over more waves.  A launch of 1 to 20 tasks takes 130 us undivided and 24 us in
 // 32 parts; at 2048 tasks and more one part each is as fast, with a count per source.
 constexpr int64_t kApplySplitWaves = 2048;
 constexpr int kApplySplitMax = 32;
