@@ -1310,6 +1310,7 @@ struct CFArgs {
   double* spec_out;
   int q0;          // first spectrum of this launch (grids hold at most 65535 rows)
   int tile;        // chains staged in LDS at a time
+  int parts;       // SPLIT: thread groups of 64 that share a tile's chains
 };
 
 // 1/d for the continued fraction: conj(d) / |d|^2 with a Newton-refined
@@ -1324,10 +1325,20 @@ __device__ __forceinline__ double2 cf_recip(double2 d) {
 // The workgroup's threads share the spectrum, so its chains' alpha and beta^2
 // are staged in LDS, a.tile chains at a time, and every level of a thread's
 // recurrence reads them there (a broadcast) instead of from memory.
-__global__ __launch_bounds__(256) void cf_kernel(CFArgs a) {
-  extern __shared__ double2 ab[];  // [a.tile][a.K]: (alpha_i, beta_i^2)
+//
+// What bounds it: one thread's recurrence is a serial chain of ~140 cycles a level.
+// SPLIT, for launches that leave the chip idle: 64 energies per workgroup and a
+// wave for every a.parts-th chain of the tile; the values meet in LDS and are summed
+// in chain order by the same expression, so the bits are the same.  One spectrum of
+// 9 chains of 100 levels, 401 energies: 64 -> 17 us; 23 spectra of 9 chains: 162 -> 65 us.
+template <bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 1024 : 256) void cf_kernel(CFArgs a) {
+  extern __shared__ double2 ab[];  // [a.tile][a.K]: (alpha_i, beta_i^2); SPLIT: then [a.tile][64] values
+  double* part_y = reinterpret_cast<double*>(ab + (size_t)a.tile * a.K);
   const int q = a.q0 + blockIdx.y;
-  const int iw = blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int part = SPLIT ? threadIdx.x >> 6 : 0, parts = SPLIT ? a.parts : 1;
+  const int iw = SPLIT ? blockIdx.x * 64 + lane : blockIdx.x * blockDim.x + threadIdx.x;
   const bool act = iw < a.n_w;
   const double om = act ? a.omega[iw] : 0.0;
   const int t0 = a.spec_chain_off[q], t1 = a.spec_chain_off[q + 1];
@@ -1349,8 +1360,7 @@ __global__ __launch_bounds__(256) void cf_kernel(CFArgs a) {
       ab[idx] = make_double2(a.alpha[c * a.K + i], b * b);
     }
     __syncthreads();
-    if (!act) continue;
-    for (int t = 0; t < nt; ++t) {
+    for (int t = part; act && t < nt; t += parts) {
       const int c = a.spec_chains[tb + t];
       const int K = a.kout[c];
       const double sg = (double)a.sign[c];
@@ -1369,10 +1379,18 @@ __global__ __launch_bounds__(256) void cf_kernel(CFArgs a) {
       const double f = sg * a.norm2[c];
       const double2 gs = make_double2(f * g.x, f * g.y);
       if (a.g_out) a.g_out[(size_t)c * a.n_w + iw] = gs;
-      acc += exp(-(a.energy[c] - emin) / kT) * (-gs.y);
+      if constexpr (SPLIT)
+        part_y[t * 64 + lane] = gs.y;
+      else
+        acc += exp(-(a.energy[c] - emin) / kT) * (-gs.y);
+    }
+    if constexpr (SPLIT) {
+      __syncthreads();
+      for (int t = 0; act && part == 0 && t < nt; ++t)
+        acc += exp(-(a.energy[a.spec_chains[tb + t]] - emin) / kT) * (-part_y[t * 64 + lane]);
     }
   }
-  if (act) a.spec_out[(size_t)q * a.n_w + iw] = Z > 0.0 ? acc / Z : 0.0;
+  if (act && part == 0) a.spec_out[(size_t)q * a.n_w + iw] = Z > 0.0 ? acc / Z : 0.0;
 }
 
 // ------------------------------------------------------------------ flat (multi-workgroup) Krylov
@@ -2544,18 +2562,30 @@ void run_cf(int C, int K, const double* alpha, const double* beta, const int32_t
     throw HipError{"continued fraction: at most 9600 Lanczos levels per chain"};
   int max_chains = 1;
   for (int q = 0; q < n_spec; ++q) max_chains = std::max(max_chains, off[q + 1] - off[q]);
-  a.tile = (int)std::max<int64_t>(1, std::min<int64_t>(max_chains, (56 * 1024) / ((int64_t)K * 16)));
-  const size_t shm = (size_t)a.tile * K * sizeof(double2);
+  // waves per 64 energies: the spectrum's chains side by side while the launch has
+  // no more than four waves per SIMD that way.  97 spectra of 9 chains, four waves
+  // each: 70 -> 65 us; 2048 spectra fill the chip with one thread an energy (690 us)
+  const int64_t wide = (int64_t)blocks_for(n_w, 64) * n_spec;
+  a.parts = 1;
+  while (a.parts < max_chains && a.parts < 16 && wide * a.parts * 2 <= 16 * (int64_t)device_cus()) a.parts *= 2;
+  const bool split = a.parts > 1;
+  const int64_t row = (int64_t)K * 16 + (split ? 64 * 8 : 0);  // LDS bytes per chain
+  a.tile = (int)std::max<int64_t>(1, std::min<int64_t>(max_chains, (56 * 1024) / row));
+  const size_t shm = (size_t)a.tile * row;
   static std::once_flag big_lds;
   std::call_once(big_lds, [] {
-    HIP_CHECK(hipFuncSetAttribute((const void*)cf_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
+    for (const void* f : {(const void*)cf_kernel<false>, (const void*)cf_kernel<true>})
+      HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 151 * 1024));
   });
   if (n_spec > 0 && n_w > 0) {
     TimedLaunch tl("cf", s);
     for (int q0 = 0; q0 < n_spec; q0 += 65535) {
       a.q0 = q0;
       const unsigned rows = (unsigned)std::min(65535, n_spec - q0);
-      hipLaunchKernelGGL(cf_kernel, dim3(blocks_for(n_w, 256), rows), dim3(256), shm, s, a);
+      if (split)
+        hipLaunchKernelGGL(cf_kernel<true>, dim3(blocks_for(n_w, 64), rows), dim3(64 * a.parts), shm, s, a);
+      else
+        hipLaunchKernelGGL(cf_kernel<false>, dim3(blocks_for(n_w, 256), rows), dim3(256), shm, s, a);
       HIP_CHECK(hipGetLastError());
     }
   }
