@@ -28,3 +28,19 @@ def gpu():
     assert torch.cuda.is_available(), "GPU tests need a GPU"
     torch.cuda.set_device(0)
     return 0
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _oracle_blas_threads(request):
+    """The oracle's golden-run chains are unconverged plain recurrences, whose last
+    printed digit depends on how the BLAS splits a dot product over threads: one
+    thread gives the same digits whatever the number of CPUs."""
+    if request.module.__name__ != "test_refout_oracle":
+        yield
+        return
+    import numpy  # noqa: F401  (the BLAS to limit)
+    import scipy.linalg  # noqa: F401
+    from threadpoolctl import threadpool_limits
+
+    with threadpool_limits(1, user_api="blas"):
+        yield
