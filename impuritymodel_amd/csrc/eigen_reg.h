@@ -220,7 +220,7 @@ bool launch_eigen(EigenArgs a, unsigned nb, int n_cu, bool test, hipStream_t s) 
   const size_t vec = (size_t)a.nmax * sizeof(T) * G;
   const int want = std::max(0, (L + G - 1) / G - Basis::S);
   const int cap = a.kl;  // eigen_lds_vectors
-  a.kl = share > fixed ? (int)std::min<size_t>(want, (share - fixed) / vec) : 0;
+  a.kl = want > 0 && share > fixed ? (int)std::min<size_t>(want, (share - fixed) / vec) : 0;
   if (cap >= 0) a.kl = std::min(a.kl, cap);
   if (a.kl < want) a.kl = a.kl / Basis::B * Basis::B;  // whole batches where vectors follow in memory
   hipLaunchKernelGGL((eigen_reg_kernel<NQ, G, R, T>), dim3(nb), dim3(64 * NQ * G), fixed + vec * a.kl, s, a);

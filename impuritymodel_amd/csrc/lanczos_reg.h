@@ -142,7 +142,8 @@ void launch_reg(LanczosArgs a, unsigned nb, int n_cu, hipStream_t s) {
   const size_t share = (size_t)kRegLds / per_cu / 1280 * 1280;
   const size_t vec = (size_t)a.nmax * sizeof(T) * G;
   const int want = std::max(0, (K - 1 + G - 1) / G - Basis::S);  // the last vector is never read
-  a.kl = share > fixed ? (int)std::min<size_t>(want, (share - fixed) / vec) : 0;
+  // want = 0 covers launches of empty chains only (vec = 0)
+  a.kl = want > 0 && share > fixed ? (int)std::min<size_t>(want, (share - fixed) / vec) : 0;
   if (a.kl < want) a.kl = a.kl / Basis::B * Basis::B;  // whole batches where vectors follow in memory
   const size_t bytes = fixed + vec * a.kl;
   if (bytes > (size_t)kRegLds) throw HipError{"lanczos: coefficients exceed the LDS"};

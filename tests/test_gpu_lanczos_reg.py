@@ -100,3 +100,19 @@ def test_register_lanczos_breakdown_and_empty_chain(gpu):
     assert (kout[0], status[0], alpha[0, 0]) == (1, IMPED_ERR_BREAKDOWN, 3.0)
     assert (kout[1], status[1]) == (10, 0)
     assert (kout[2], status[2]) == (0, 0)
+
+
+@pytest.mark.parametrize("complex_h", [True, False])
+@pytest.mark.parametrize("n_empty,others", [(1, 0), (3, 0), (1, 300), (2, 300)])
+def test_register_lanczos_launch_of_empty_chains_only(gpu, complex_h, n_empty, others):
+    # no state in any chain of a launch: alone, and beside more chains of 70 rows
+    # than the chip has CUs (the classes then launch separately)
+    empty = (scipy.sparse.csr_matrix((0, 0), dtype=complex), np.zeros(0, complex))
+    chain = _chain(np.random.default_rng(7), 70, complex_h, "complex" if complex_h else "real")
+    alpha, _, kout, status = _run([empty] * n_empty + [chain] * others, 12)
+    assert not kout[:n_empty].any() and not status[:n_empty].any()
+    if others:
+        a, _ = _lanczos(*chain, 12)
+        assert (kout[n_empty:] == 12).all() and not status[n_empty:].any()
+        scale = max(1.0, abs(chain[0]).sum(axis=1).max())
+        assert np.abs(alpha[n_empty:] - a).max() <= 1e-10 * scale
