@@ -10,7 +10,10 @@
 // * gather_kernel, loss_sum_kernel: minibatch inputs and the losses.
 //
 // BF16 copies of weights and activations are stored with rows padded to a
-// multiple of 64 entries, the padding zero, so no load is bounds-checked.
+// multiple of 64 entries, the padding zero, so no load is bounds-checked.  The
+// epilogues write those zeros whatever the sum is: an infinite activation times
+// a padding row of weights is NaN, and one NaN in the padding of a row would
+// reach every output of its sample (or, from a padding sample, every weight).
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -250,6 +253,7 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(NtArgs g) {
     // first store: first used inside the per-row branches, it would put a wait
     // for every earlier store between the stores
     const float bn = n < g.N ? g.bias[(int64_t)z * g.bias_z + n] : 0.0f;
+    const uint16_t col = n < g.N ? 0xffff : 0;  // a mask, not a branch around the GELU
     float v[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -260,7 +264,7 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(NtArgs g) {
     for (int r = 0; r < 16; ++r) {
       const int m = mb + 8 * (r >> 2) + (r & 3);
       if constexpr (EPI == NT_HIDDEN)
-        g.C[((int64_t)z * g.mp + m) * g.np + n] = f2bf(gelu_inference(v[r]));
+        g.C[((int64_t)z * g.mp + m) * g.np + n] = f2bf(gelu_inference(v[r])) & col;
       else if (m < g.M && n < g.N)
         g.out[((int64_t)z * g.M + m) * g.N + n] = v[r];
     }
@@ -277,14 +281,15 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(NtArgs g) {
         const int m = mb + 8 * q + r;
         const int64_t o = cz + (int64_t)m * g.np + n;
         const float v = acc[4 * q + r] + bn;
+        const bool data = m < g.M && n < g.N;
+        h[r] = 0;
         if constexpr (EPI == NT_GELU) {
           g.z[o] = v;
-          h[r] = f2bf(gelu(v));
+          h[r] = data ? f2bf(gelu(v)) : (uint16_t)0;
         } else if constexpr (EPI == NT_DGELU) {
-          h[r] = f2bf(v * gelu_grad(g.z[o]));
+          h[r] = data ? f2bf(v * gelu_grad(g.z[o])) : (uint16_t)0;
         } else {
-          h[r] = 0;
-          if (m < g.M && n < g.N) {
+          if (data) {
             const float d = v - g.T[(int64_t)(g.idx ? g.idx[m] : m) * g.N + n];
             h[r] = f2bf(2.0f * d / (float)((int64_t)g.M * g.N));
             sq += (double)d * (double)d;

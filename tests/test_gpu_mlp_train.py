@@ -52,3 +52,78 @@ def test_fused_adam_steps_match_numpy(gpu, dims, batch):
     # error is that of the gradient, elsewhere a few ulp; 1e-5 of lr holds both
     assert np.quantile(np.abs(got - p), 0.999) <= 1e-5 * lr + 2e-7 * np.abs(p).max()
     assert np.abs(got - p).max() <= 2e-2 * lr
+
+
+def _layer_views(p, dims):
+    """Views (weights [members, out, in], biases [members, out]) of flat parameters, by layer."""
+    out, off = [], 0
+    for l in range(len(dims) - 1):
+        i, o = dims[l], dims[l + 1]
+        out.append((p[:, off:off + o * i].reshape(len(p), o, i), p[:, off + o * i:off + o * i + o]))
+        off += o * i + o
+    return out
+
+
+@pytest.mark.parametrize("dims", [(8, 100, 72, 70), (5, 100, 72, 70), (8, 64, 128, 64)])
+def test_infinite_activations_stay_in_their_sample(gpu, dims):
+    """One hidden unit of one sample overflows: with positive weights behind it every output of
+    that sample is +inf (no product is inf * 0 or inf - inf), the other samples are those of the
+    network without that unit's weight, bit for bit."""
+    from impuritymodel_amd.surrogate import Ensemble
+
+    net = Ensemble(2, dims, max_batch=8, seed=3)
+    plain = np.abs(net.init_params(9)) + np.float32(1e-3)
+    plain[:, sum(dims[l + 1] * (dims[l] + 1) for l in range(3)):] = 0.0
+    for _, b in _layer_views(plain, dims):
+        b[:] = 0.0
+    _layer_views(plain, dims)[0][0][:, 7, 0] = 0.0
+    huge = plain.copy()
+    _layer_views(huge, dims)[0][0][:, 7, 0] = 2.0 ** 127
+    x = np.random.default_rng(2).uniform(0.1, 1, (6, dims[0])).astype(np.float32)
+    x[:, 0] = 0.0
+    net.set_params(plain)
+    want = net.forward(x)
+    x[2, 0] = 4.0
+    net.set_params(huge)
+    got = net.forward(x)
+    keep = np.arange(6) != 2
+    assert np.array_equal(got[:, keep], want[:, keep]) and np.all(np.isfinite(got[:, keep]))
+    assert np.all(got[:, 2] == np.inf)
+    # the same through the training pass: the sample's losses and gradients are not finite,
+    # so it is the forward's other samples alone that can be compared: leave it out
+    g0 = net.gradients(x[keep], want[0, keep])
+    net.set_params(plain)
+    g1 = net.gradients(x[keep], want[0, keep])
+    assert np.array_equal(g0[0], g1[0]) and np.all(np.isfinite(g0[1]))
+    for l, ((w0, b0), (w1, b1)) in enumerate(zip(_layer_views(g0[1], dims), _layer_views(g1[1], dims))):
+        assert np.array_equal(w0, w1) and np.array_equal(b0, b1), l
+
+
+@pytest.mark.parametrize("dims,batch", [((8, 100, 72, 70), 3), ((8, 64, 64, 64), 65)])
+def test_gradients_with_overflow_in_the_padding_samples(gpu, dims, batch):
+    """A bias of 2^127 that every sample cancels exactly: z = 0 for the batch, while the rows that
+    pad the batch to whole tiles overflow in the second layer.  Losses and gradients are those of
+    the network without the bias and the weight, bit for bit."""
+    from impuritymodel_amd.surrogate import Ensemble
+
+    net = Ensemble(2, dims, max_batch=8, seed=3)
+    rng = np.random.default_rng(5)
+    plain = net.init_params(9)
+    views = _layer_views(plain, dims)
+    views[0][0][:, 7, :] = 0.0
+    views[0][1][:, 7] = 0.0
+    views[1][0][:, :, 7] = 4.0
+    big = plain.copy()
+    views = _layer_views(big, dims)
+    views[0][0][:, 7, 0] = -(2.0 ** 127)
+    views[0][1][:, 7] = 2.0 ** 127
+    x = rng.uniform(-1, 1, (batch, dims[0])).astype(np.float32)
+    x[:, 0] = 1.0
+    t = rng.normal(size=(batch, dims[-1])).astype(np.float32)
+    net.set_params(plain)
+    want_loss, want = net.gradients(x, t)
+    net.set_params(big)
+    loss, got = net.gradients(x, t)
+    assert np.all(np.isfinite(want)) and np.array_equal(loss, want_loss) and np.array_equal(got, want)
+    p = [net.train(x, t, epochs=1, batch=batch, lr=1e-3), net.get_params()]
+    assert np.all(np.isfinite(p[0])) and np.all(np.isfinite(p[1]))
