@@ -92,21 +92,27 @@ def applyOp(n_spin_orbitals, op, psi, slaterWeightMin=1e-12, restrictions=None, 
         k, a, _ = out.get()
         return dict(zip(opcompile.words_to_bytes(k, n), a.tolist()))
     new_states = [s for s in psi if s not in opResult]
-    return _memo_sum(psi, _state_results(n, ops, 1, new_states)[0], slaterWeightMin, opResult)
+    return _memo_sum(psi, next(_state_results(n, ops, 1, new_states)), slaterWeightMin, opResult)
 
 
 def _state_results(n, ops, n_models, states):
-    """Per model of ``ops`` a dict {state: [(target, value), ...]}, the targets in
-    the operator's order and unpruned, from one batched application."""
+    """For each model of ``ops`` in turn a dict {state: [(target, value), ...]}, the
+    targets in the operator's order and unpruned, from one batched application.
+    The arrays of all models are held, Python objects of one model at a time."""
     if not states:
-        return [{} for _ in range(n_models)]
+        for _ in range(n_models):
+            yield {}
+        return
     ns = len(states)
     src = Vec(ops.W, keys=_words(states, n), amps=np.ones(ns, complex), offsets=np.arange(ns + 1, dtype=np.int64))
     out = vec_apply(ops, src, np.tile(np.arange(ns), n_models), np.repeat(np.arange(n_models), ns), 0.0)
     k, a, _ = out.get()
-    off = out.offsets.tolist()
-    entries = list(zip(opcompile.words_to_bytes(k, n), a.tolist()))
-    return [{s: entries[off[m * ns + i]:off[m * ns + i + 1]] for i, s in enumerate(states)} for m in range(n_models)]
+    offsets = out.offsets
+    for m in range(n_models):
+        off = offsets[m * ns:(m + 1) * ns + 1]
+        entries = list(zip(opcompile.words_to_bytes(k[off[0]:off[-1]], n), a[off[0]:off[-1]].tolist()))
+        off = (off - off[0]).tolist()
+        yield {s: entries[off[i]:off[i + 1]] for i, s in enumerate(states)}
 
 
 def _memo_sum(psi, per_state, slaterWeightMin, opResult):

@@ -60,7 +60,8 @@ def getGreen(n_spin_orbitals, e, psi, hOp, omega, delta, krylovSize, slaterWeigh
     return g[0]
 
 
-_MEMO_VECTORS = 1 << 20  # result vectors of one batched application at most
+_MEMO_VECTORS = 1 << 20  # result vectors of one batched application at most,
+_MEMO_ENTRIES = 1 << 22  # and their entries: a state has at most one per term of the operator
 
 
 def _transition_states_memo(n, tOps, psis, slaterWeightMin, restrictions):
@@ -74,12 +75,16 @@ def _transition_states_memo(n, tOps, psis, slaterWeightMin, restrictions):
     states = list(dict.fromkeys(s for psi in psis for s in psi))
     # operators applied per launch: every state under all of them at once (20
     # operators on 150 states: 60 applications one by one took 25 ms, this 1 ms),
-    # fewer when the states alone fill one
-    step = max(1, _MEMO_VECTORS // max(len(states), 1))
+    # fewer when the states of one alone fill it
+    parts = []
+    for tOp in tOps:
+        if (not parts or len(states) * (len(parts[-1]) + 1) > _MEMO_VECTORS
+                or len(states) * sum(map(len, [*parts[-1], tOp])) > _MEMO_ENTRIES):
+            parts.append([])
+        parts[-1].append(tOp)
     keys, amps = [], []
-    for t0 in range(0, len(tOps), step):
-        part = list(tOps[t0:t0 + step])
-        ops = Ops(part, [restrictions] * len(part), n, W)
+    for part in parts:
+        ops = Ops(part, [restrictions] * len(part), n, W) if states else None
         for per_state in _state_results(n, ops, len(part), states):
             t_big = {}
             for psi in psis:
@@ -87,6 +92,7 @@ def _transition_states_memo(n, tOps, psis, slaterWeightMin, restrictions):
                 ks = list(psiR.keys())
                 keys.append(_words(ks, n) if ks else np.zeros((0, W), np.uint64))
                 amps.append(np.array([complex(x) for x in psiR.values()], np.complex128))
+            del per_state, t_big  # one operator's results at a time
     return keys, amps
 
 

@@ -135,3 +135,60 @@ def test_c_abi_rejects_null_arguments():
     assert lib.imped_batch_seed_affine(None, None, None, None, None, None, 0.0, 0.0, None) == IMPED_ERR_INVALID
     assert lib.imped_family_xas(None, None, None, 1, 1, None, 0, None, None, 1, 1, 1.0, 1, 1, 1e-12, 10, 0, 0.0, 0.0,
                                 0.0, None, 0, 0.1, None, None, None, None, None, None, None) == IMPED_ERR_INVALID
+
+
+def test_batched_transition_states_hold_one_operators_objects(monkeypatch):
+    """The memo of several operators over one application (here a stand-in that gives every
+    state 30 targets): Python objects of one operator at a time, the arrays of a launch bounded."""
+    import tracemalloc
+
+    from impuritymodel_amd import finite, spectra
+
+    n, targets, sizes = 40, 30, []
+
+    class StubOps:
+        def __init__(self, ops, restrictions, n_orb, W=None):
+            self.W = W
+
+    class StubVec:
+        def __init__(self, W, keys=None, amps=None, offsets=None):
+            self.keys, self.amps, self.offsets = keys, amps, offsets
+
+        def get(self):
+            return self.keys, self.amps, None
+
+    def stub_apply(ops, src, vectors, models, weight_min):
+        sizes.append((len(vectors), len(vectors) * targets))
+        keys = src.keys[vectors].repeat(targets, axis=0) ^ (np.arange(targets, dtype=np.uint64) << np.uint64(40)).repeat(
+            len(vectors)).reshape(targets, -1).T.reshape(-1, 1)
+        return StubVec(1, keys, np.ones(len(keys), complex), np.arange(len(vectors) + 1) * targets)
+
+    monkeypatch.setattr(finite, "Vec", StubVec)
+    monkeypatch.setattr(finite, "vec_apply", stub_apply)
+    monkeypatch.setattr(spectra, "Ops", StubOps)
+    rng = np.random.default_rng(1)
+    states = opcompile.words_to_bytes(rng.integers(0, 1 << 30, 1500, dtype=np.uint64)[:, None] << np.uint64(26), n)
+    psi = {s: 1.0 + 0.0j for s in states}
+
+    def peak(n_op):
+        op = dict.fromkeys(range(targets), 1.0)
+        tracemalloc.start()
+        keys, amps = spectra._transition_states_memo(n, [op] * n_op, [psi], 2.0, None)
+        top = tracemalloc.get_traced_memory()[1] - sum(k.nbytes + a.nbytes for k, a in zip(keys, amps))
+        tracemalloc.stop()
+        assert len(keys) == n_op
+        return top
+
+    one = peak(1)
+    # an operator's arrays are 24 bytes an entry beside over 200 of its Python objects
+    assert peak(12) < 12 * 1500 * targets * 60 + 1.5 * one
+    sizes.clear()
+    monkeypatch.setattr(spectra, "_MEMO_ENTRIES", 4 * 1500 * targets)
+    peak(10)
+    assert [v for v, _ in sizes] == [6000, 6000, 3000] and all(e <= spectra._MEMO_ENTRIES for _, e in sizes)
+    monkeypatch.setattr(spectra, "_MEMO_VECTORS", 3000)
+    sizes.clear()
+    peak(3)
+    assert [v for v, _ in sizes] == [3000, 1500]
+    assert spectra._transition_states_memo(n, [], [psi], 2.0, None) == ([], [])
+    assert [len(k) for k in spectra._transition_states_memo(n, [{}], [{}, {}], 2.0, None)[0]] == [0, 0]
