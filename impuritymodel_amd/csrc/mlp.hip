@@ -1014,20 +1014,24 @@ void mlp_train(Mlp& net, const int32_t* batches, int steps, int B, float lr, flo
   DevBuf didx, lossp, lbuf;
   h2d(didx, batches, (size_t)steps * B, s);
   const int tiles = loss_tiles(net, B);
-  const int n_loss = std::max(steps, 1) * net.E;
-  lossp.reserve((size_t)n_loss * tiles * 8);
-  lbuf.reserve((size_t)n_loss * 8);
+  // the tiles' sums of squares of up to 1 MiB of steps, summed into lbuf before
+  // the next steps overwrite them
+  const size_t step_bytes = (size_t)net.E * tiles * 8;
+  const int group = (int)std::max<size_t>(1, std::min<size_t>(steps, (size_t(1) << 20) / step_bytes));
+  lossp.reserve(group * step_bytes);
+  lbuf.reserve((size_t)std::max(steps, 1) * net.E * 8);
   for (int it = 0; it < steps; ++it) {
     const int32_t* idx = didx.as<int32_t>() + (size_t)it * B;
     gather_batch(net, net.dX.as<float>(), idx, B, s);
     ++net.step;
     const AdamStep adam{lr, b1, b2, eps, 1.0f - powf(b1, (float)net.step), 1.0f - powf(b2, (float)net.step)};
-    train_pass(net, B, net.dY.as<float>(), idx, lossp.as<double>() + (size_t)it * net.E * tiles, &adam, s);
-  }
-  if (steps > 0) {
-    hipLaunchKernelGGL(loss_sum_kernel, dim3(steps * net.E), dim3(64), 0, s, lossp.as<double>(), tiles,
-                       (double)B * net.dims[net.L], lbuf.as<double>());
-    HIP_CHECK(hipGetLastError());
+    const int k = it % group;
+    train_pass(net, B, net.dY.as<float>(), idx, lossp.as<double>() + (size_t)k * net.E * tiles, &adam, s);
+    if (k + 1 == group || it + 1 == steps) {
+      hipLaunchKernelGGL(loss_sum_kernel, dim3((k + 1) * net.E), dim3(64), 0, s, lossp.as<double>(), tiles,
+                         (double)B * net.dims[net.L], lbuf.as<double>() + (size_t)(it - k) * net.E);
+      HIP_CHECK(hipGetLastError());
+    }
   }
   if (losses) d2h(losses, lbuf.p, (size_t)steps * net.E, s);
   stream_sync(s);

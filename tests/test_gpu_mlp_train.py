@@ -127,3 +127,19 @@ def test_gradients_with_overflow_in_the_padding_samples(gpu, dims, batch):
     assert np.all(np.isfinite(want)) and np.array_equal(loss, want_loss) and np.array_equal(got, want)
     p = [net.train(x, t, epochs=1, batch=batch, lr=1e-3), net.get_params()]
     assert np.all(np.isfinite(p[0])) and np.all(np.isfinite(p[1]))
+
+
+def test_losses_of_many_steps_in_one_call(gpu):
+    """More steps in one call than the partial sums are kept for (256 at this size): the same
+    losses and weights as in calls of 100 steps, bit for bit (constant learning rate)."""
+    from impuritymodel_amd.surrogate import Ensemble
+
+    rng = np.random.default_rng(8)
+    x = rng.uniform(-1, 1, (512, 4)).astype(np.float32)
+    t = rng.normal(size=(512, 2048)).astype(np.float32)
+    out = []
+    for chunk in (100, 600):
+        net = Ensemble(2, (4, 2048), max_batch=512, seed=3)
+        out.append((net.train(x, t, epochs=600, batch=512, lr=1e-3, seed=4, chunk=chunk), net.get_params()))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert np.all(out[0][0] > 0) and np.all(out[0][0][-1] < out[0][0][0])
