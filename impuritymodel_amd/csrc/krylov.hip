@@ -24,6 +24,7 @@
 #include "krylov.h"
 #include "krylov_reg.h"
 #include "krylov_ritz.h"
+#include "orth_estimate.h"
 
 namespace imped {
 
@@ -439,60 +440,6 @@ __device__ __forceinline__ double update_basis(const T* V, int m, int64_t n, T* 
   }
   return block_sum<BT>(p, red);
 }
-
-// Estimates of the inner products <v_j, v_k>, k < j, of the Lanczos vectors of
-// one chain from its recurrence coefficients alone (H. D. Simon, "The Lanczos
-// algorithm with partial reorthogonalization", Math. Comp. 42, 1984):
-//   b_j w_{j+1,k} = b_k w_{j,k+1} + (a_k - a_j) w_{j,k} + b_{k-1} w_{j,k-1}
-//                   - b_{j-1} w_{j-1,k} + rounding of order eps (b_k + b_j).
-// The basis then needs a Gram-Schmidt pass only in the steps where an estimate
-// passes kOrthLevel (and in the step after, since two vectors feed the next
-// one).  Simon's level sqrt(eps) keeps the eigenvalues at eps |H|, but Ritz
-// vectors formed as V y then carry errors of that level times y: at 1e-13 their
-// residuals are those of full reorthogonalization.  Measured in 64-bit numpy on
-// sectors of 1770 and 1225 states (200 and 300 steps), residuals of the two
-// lowest pairs: full 0.3 to 2.2e-12, level 1e-13 0.4 to 2.3e-12 with 18 and 22%
-// of the vector reads, level 1e-11 up to 2e-11, sqrt(eps) up to 9e-8.
-// On one MI355X, 2.9e6 states (252 steps): 252 -> 42 passes over the basis, which is
-// read at 4.6 TB/s either way, 299 -> 55 ms; the whole spectrum of that instance
-// 419 -> 214 ms.
-constexpr double kOrthLevel = 1e-13;
-
-struct OrthEstimate {
-  std::vector<double> w, w_old, next;  // w[k] of the latest vector, of the one before, and work
-  std::vector<double> a, b;
-  bool again = false;                  // the step after a pass
-
-  OrthEstimate() : w{1.0} {}
-  // After step j's three-term update (alpha_j = al, |w| = bt): whether
-  // v_{j+1} needs a pass against v_0..v_j.
-  bool step(double al, double bt) {
-    const int j = (int)a.size();
-    a.push_back(al);
-    next.assign(j + 2, 0.0);
-    next[j + 1] = 1.0;
-    double worst = 0.0;
-    for (int k = 0; k < j; ++k) {
-      double t = b[k] * w[k + 1] + (a[k] - al) * w[k] - b[j - 1] * w_old[k];
-      if (k > 0) t += b[k - 1] * w[k - 1];
-      t += std::copysign(4.4e-16 * (b[k] + bt), t);
-      next[k] = t / bt;
-      worst = std::max(worst, std::fabs(next[k]));
-    }
-    next[j] = 2.2e-16 * (std::fabs(al) + bt + (j > 0 ? b[j - 1] : 0.0)) / bt;  // rounding of alpha_j
-    worst = std::max(worst, std::fabs(next[j]));
-    const bool pass = again || !(worst <= kOrthLevel) || !(bt > 0.0);
-    again = pass && !again;
-    return pass;
-  }
-  // beta_j as it came out; the estimates move on to v_{j+1}
-  void done(double bt, bool passed) {
-    if (passed) std::fill(next.begin(), next.end() - 1, 2.2e-16);
-    b.push_back(bt);
-    w_old.swap(w);
-    w.swap(next);
-  }
-};
 
 // LW: the tridiagonal and the Ritz work arrays live in LDS (a compile-time
 // choice, so every access to them is an LDS instruction), else in memory.
@@ -1406,10 +1353,12 @@ __global__ __launch_bounds__(SPLIT ? 1024 : 256) void cf_kernel(CFArgs a) {
 constexpr int FT = 256;  // threads per flat block
 
 // VR: the values are real and read from vre (8 bytes each) instead of val.
-template <int LPR, class T, bool VR = false>
+// SH: y = (H - sigma) x, sigma taken off the diagonal entry itself, so that no
+// rounding of order eps |sigma| enters (it would, taken off H x).
+template <int LPR, class T, bool VR = false, bool SH = false>
 __device__ __forceinline__ void spmv_rows(const int64_t* rowptr, const int32_t* col, const double2* val, int64_t base,
                                           int64_t n, const T* x, T* y, double* partial, double* red,
-                                          const double* vre = nullptr) {
+                                          const double* vre = nullptr, double sigma = 0.0) {
   const int g = threadIdx.x / LPR, r = threadIdx.x % LPR;
   double pa = 0.0;
   // grid-stride over groups of FT/LPR rows, so the partial sums number at
@@ -1417,16 +1366,26 @@ __device__ __forceinline__ void spmv_rows(const int64_t* rowptr, const int32_t* 
   for (int64_t rb = blockIdx.x; rb * (FT / LPR) < n; rb += gridDim.x) {
     const int64_t row = rb * (FT / LPR) + g;
     double ax = 0.0, ay = 0.0;
+    bool shifted = false;  // SH: this lane has met the diagonal entry
     if (row < n) {
       const int64_t e0 = rowptr[base + row], e1 = rowptr[base + row + 1];
       for (int64_t e = e0 + r; e < e1; e += LPR) {
-        const T v = x[col[e]];
+        const int32_t c = col[e];
+        const T v = x[c];
         if constexpr (VR) {
-          const double h = vre[e];
+          double h = vre[e];
+          if constexpr (SH) {
+            h -= c == row && !shifted ? sigma : 0.0;
+            shifted = shifted || c == row;
+          }
           ax += h * re_(v);
           if constexpr (!is_real_v<T>) ay += h * im_(v);
         } else {
-          const double2 h = val[e];
+          double2 h = val[e];
+          if constexpr (SH) {
+            h.x -= c == row && !shifted ? sigma : 0.0;
+            shifted = shifted || c == row;
+          }
           if constexpr (is_real_v<T>) {
             ax += h.x * re_(v);
           } else {
@@ -1441,7 +1400,16 @@ __device__ __forceinline__ void spmv_rows(const int64_t* rowptr, const int32_t* 
       ax += __shfl_xor(ax, off);
       if constexpr (!is_real_v<T>) ay += __shfl_xor(ay, off);
     }
+    [[maybe_unused]] int times = 1;  // SH: lanes of this row that took sigma off (0: no diagonal entry)
+    if constexpr (SH) {
+      const uint64_t row_lanes = LPR == 64 ? ~0ull : (1ull << (LPR & 63)) - 1;
+      times = __popcll((__ballot(shifted) >> (threadIdx.x & 63 & ~(LPR - 1))) & row_lanes);
+    }
     if (row < n && r == 0) {
+      if (SH && times != 1) {
+        ax += (times - 1) * sigma * re_(x[row]);
+        ay += (times - 1) * sigma * im_(x[row]);
+      }
       y[row] = mk<T>(ax, ay);
       pa += ax * re_(x[row]) + ay * im_(x[row]);
     }
@@ -1453,9 +1421,9 @@ __device__ __forceinline__ void spmv_rows(const int64_t* rowptr, const int32_t* 
 template <int LPR, class T, bool VR>
 __global__ __launch_bounds__(FT) void flat_spmv_kernel(const int64_t* rowptr, const int32_t* col, const double2* val,
                                                        const double* vre, int64_t base, int64_t n, const T* x, T* y,
-                                                       double* partial) {
+                                                       double* partial, double sigma) {
   __shared__ double red[FT / 64];
-  spmv_rows<LPR, T, VR>(rowptr, col, val, base, n, x, y, partial, red, vre);
+  spmv_rows<LPR, T, VR, true>(rowptr, col, val, base, n, x, y, partial, red, vre, sigma);
 }
 
 // out[k] = sum of partial[k*stride .. k*stride + count) in a fixed order;
@@ -1611,12 +1579,13 @@ __global__ void flat_set_beta_kernel(const double* p, double* beta_j, double* sc
   }
 }
 
-// Ritz check of T_m (one workgroup): eigenvalues, inverse-iteration vectors,
-// residuals |beta_m y_k[m-1]| against tol; flags convergence.
-__global__ __launch_bounds__(FT) void flat_ritz_kernel(const double* alpha, const double* beta, int m, int nev,
-                                                       double tol, int ms, double* evals, double* Y, double* tw,
+// Ritz check of T_m, the tridiagonal of H - sigma (one workgroup): eigenvalues
+// of H, inverse-iteration vectors, residuals |beta_m y_k[m-1]| against tol;
+// flags convergence.
+__global__ __launch_bounds__(FT) void flat_ritz_kernel(const double* alpha, const double* beta, double sigma, int m,
+                                                       int nev, double tol, int ms, double* evals, double* Y, double* tw,
                                                        int* tpiv, int32_t* converged, uint64_t seed) {
-  __shared__ double s_lam[MAX_NEV], s_lo[MAX_NEV], s_hi[MAX_NEV];
+  __shared__ double s_lam[MAX_NEV], s_energy[MAX_NEV], s_lo[MAX_NEV], s_hi[MAX_NEV];
   __shared__ int s_first[MAX_NEV];
   __shared__ int s_flag, s_done;
   const int ne = nev < m ? nev : m;
@@ -1629,12 +1598,13 @@ __global__ __launch_bounds__(FT) void flat_ritz_kernel(const double* alpha, cons
     double* t = tw + (size_t)k * 5 * ms;
     tri_inverse_iteration(alpha, beta, m, s_lam[k], y, t, t + ms, t + 2 * ms, t + 3 * ms, tpiv + (size_t)k * ms,
                           seed + 7919 * (uint64_t)k);
-    evals[k] = s_lam[k];
-    if (!(fabs(beta[m - 1] * y[m - 1]) <= tol * fmax(1.0, fabs(s_lam[k])))) atomicAnd(&s_done, 0);
+    s_energy[k] = s_lam[k] + sigma;
+    evals[k] = s_energy[k];
+    if (!(fabs(beta[m - 1] * y[m - 1]) <= tol * fmax(1.0, fabs(s_energy[k])))) atomicAnd(&s_done, 0);
   }
   __syncthreads();
   // orthogonalize inverse-iteration vectors of clustered eigenvalues
-  ortho_clustered(Y, ms, m, ne, s_lam);
+  ortho_clustered(Y, ms, m, ne, s_energy);
   if (threadIdx.x == 0) *converged = s_done;
 }
 
@@ -1708,19 +1678,20 @@ int64_t chain_base(const KrylovBatch& kb, int c) {
 
 unsigned vec_blocks(int64_t n) { return (unsigned)std::min<int64_t>(std::max<int64_t>((n + FT - 1) / FT, 1), 2048); }
 
+// y = (H - sigma) x, partial Re <x, y> per block
 template <class T>
-void launch_spmv(int lpr, const KrylovBatch& kb, int64_t base, int64_t n, const T* x, T* y, double* partial,
-                 unsigned* nb_out, hipStream_t s) {
+void launch_spmv(int lpr, const KrylovBatch& kb, int64_t base, int64_t n, const T* x, T* y, double sigma,
+                 double* partial, unsigned* nb_out, hipStream_t s) {
   const unsigned nb = (unsigned)std::min<int64_t>(std::max<int64_t>((n + FT / lpr - 1) / (FT / lpr), 1), 4096);
   *nb_out = nb;
   TimedLaunch tl("spmv", s);
 #define IMPED_SPMV(L)                                                                                           \
   if (kb.val_re)                                                                                               \
     hipLaunchKernelGGL((flat_spmv_kernel<L, T, true>), dim3(nb), dim3(FT), 0, s, kb.rowptr, kb.col, kb.val,     \
-                       kb.val_re, base, n, x, y, partial);                                                      \
+                       kb.val_re, base, n, x, y, partial, sigma);                                               \
   else                                                                                                         \
     hipLaunchKernelGGL((flat_spmv_kernel<L, T, false>), dim3(nb), dim3(FT), 0, s, kb.rowptr, kb.col, kb.val,    \
-                       kb.val_re, base, n, x, y, partial)
+                       kb.val_re, base, n, x, y, partial, sigma)
   switch (lpr) {
     case 4: IMPED_SPMV(4); break;
     case 8: IMPED_SPMV(8); break;
@@ -1945,9 +1916,14 @@ void lanczos_flat_chain(const KrylovBatch& kb, int c, const double2* v0, int K, 
   for (; j < Kc; ++j) launch_lanczos_step(a, nbv, nbs, lpr, kb.val_re != nullptr, s);
 }
 
-// Lowest eigenpairs of one large chain: Lanczos with the basis kept orthogonal
-// by grid-wide Gram-Schmidt passes in the steps that need one (every step, twice,
-// with eigen_dgks off), host-controlled (one small read-back per step).
+// Lowest eigenpairs of one large chain: Lanczos on H - sigma, sigma = <v_0, H v_0>
+// (orth_estimate.h), with the basis kept orthogonal by grid-wide Gram-Schmidt passes
+// in the steps that need one (every step, twice, with eigen_dgks off),
+// host-controlled (one small read-back per step and one per pass).
+//
+// On one MI355X, 2.9e6 states (252 steps): 252 -> 62 passes over the basis, which is
+// read at 4.6 TB/s either way, 299 -> 80 ms; taking sigma off the diagonal costs the
+// product 1 to 2% (139 -> 141 us).
 template <class T>
 int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_steps, uint64_t seed, double* evals,
                      double2* X, int32_t* steps_out, hipStream_t s) {
@@ -1992,11 +1968,18 @@ int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_
     hipLaunchKernelGGL(flat_reduce_kernel, dim3(1), dim3(FT), 0, s, part, (int64_t)nbv, (int64_t)0, scal + 2, 0);
     HIP_CHECK(hipGetLastError());
   };
-  OrthEstimate orth;
+  unsigned nbs = 0;
+  double sigma = 0.0;
+  launch_spmv<T>(lpr, kb, base, n, V, w, 0.0, part, &nbs, s);
+  hipLaunchKernelGGL(flat_reduce_kernel, dim3(1), dim3(FT), 0, s, part, (int64_t)nbs, (int64_t)0, scal, 0);
+  HIP_CHECK(hipGetLastError());
+  d2h_bytes(&sigma, scal, sizeof(double), s);
+  stream_sync(s);
+  if (!std::isfinite(sigma)) sigma = 0.0;
+  OrthEstimate orth(sigma);
   for (int j = 0; j < mmax; ++j) {
     const T* vj = V + (size_t)j * n;
-    unsigned nbs = 0;
-    launch_spmv<T>(lpr, kb, base, n, vj, w, part, &nbs, s);
+    launch_spmv<T>(lpr, kb, base, n, vj, w, sigma, part, &nbs, s);
     hipLaunchKernelGGL(flat_reduce_kernel, dim3(1), dim3(FT), 0, s, part, (int64_t)nbs, (int64_t)0, alpha + j, 0);
     hipLaunchKernelGGL((flat_update_kernel<T>), dim3(nbv), dim3(FT), 0, s, w, vj, j > 0 ? vj - n : (const T*)nullptr,
                        alpha + j, j > 0 ? beta + j - 1 : nullptr, n, part);
@@ -2026,9 +2009,9 @@ int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_
     hipLaunchKernelGGL(flat_set_beta_kernel, dim3(1), dim3(64), 0, s, scal + (pass ? 2 : 1), beta + j, scal + 3);
     HIP_CHECK(hipGetLastError());
     m = j + 1;
-    const bool last = (m == mmax) || b <= 1e-13 * (std::fabs(al) + bprev + 1e-300);
+    const bool last = (m == mmax) || b <= 1e-13 * (std::fabs(al + sigma) + bprev + 1e-300);
     if (last || (m >= nev && m % g_tuning.eigen_check_every == 0)) {
-      hipLaunchKernelGGL(flat_ritz_kernel, dim3(1), dim3(FT), 0, s, alpha, beta, m, nev, tol, mmax,
+      hipLaunchKernelGGL(flat_ritz_kernel, dim3(1), dim3(FT), 0, s, alpha, beta, sigma, m, nev, tol, mmax,
                          evals, sc.yk.as<double>(), sc.tw.as<double>(), sc.tpiv.as<int>(), sc.conv.as<int32_t>(),
                          seed);
       HIP_CHECK(hipGetLastError());
@@ -2050,6 +2033,18 @@ int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_
                      X, part);
   hipLaunchKernelGGL(flat_reduce_kernel, dim3(ne), dim3(FT), 0, s, part, (int64_t)nbr, (int64_t)nbr, scal + 4, 0);
   hipLaunchKernelGGL(flat_normalize_kernel, dim3(nbr), dim3(FT), 0, s, X, n, scal + 4, ne);
+  // the basis is orthogonal to kOrthLevel, the vectors to rounding
+  for (int k = 1; k < ne; ++k) {
+    double2* xk = X + (size_t)k * n;
+    hipLaunchKernelGGL((flat_dots_kernel<double2>), dim3(nbd), dim3(FT), 0, s, X, k, n, xk, sc.fcpart.as<double2>(),
+                       chunk);
+    hipLaunchKernelGGL(flat_reduce_c_kernel, dim3(k), dim3(FT), 0, s, sc.fcpart.as<double2>(), (int)nbd,
+                       sc.fcoef.as<double2>());
+    hipLaunchKernelGGL((flat_gs_update_kernel<double2>), dim3(nbr), dim3(FT), 0, s, X, k, n, xk,
+                       sc.fcoef.as<double2>(), part);
+    hipLaunchKernelGGL(flat_reduce_kernel, dim3(1), dim3(FT), 0, s, part, (int64_t)nbr, (int64_t)nbr, scal + 4, 0);
+    hipLaunchKernelGGL(flat_normalize_kernel, dim3(nbr), dim3(FT), 0, s, xk, n, scal + 4, 1);
+  }
   HIP_CHECK(hipGetLastError());
   if (ne < nev) {
     HIP_CHECK(hipMemsetAsync(X + (size_t)ne * n, 0, (size_t)(nev - ne) * n * sizeof(double2), s));
