@@ -42,6 +42,8 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
     return;
   }
   const int mmax = a.max_steps < n ? a.max_steps : n;
+  // Sturm points by the chain's size: every instance that may hold it has the threads
+  const int points = n <= 64 ? 64 : 256;
   // LDS: tridiagonal and Ritz work arrays (stride L), the residual, the basis
   const int L = a.lstride;
   double* sa = reinterpret_cast<double*>(lds);
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
     const double xi = reg_real_v<T> || !b.on[r] ? 0.0 : u01(u + 1) - 0.5;
     set1(w[r], xr, xi);
     set1(vp[r], 0.0, 0.0);
-    p += xr * xr + xi * xi;
+    p = add_re(p, w[r], w[r]);
   }
   auto publish = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
   auto ritz_check = [&](bool last, double bt) __attribute__((always_inline)) -> bool {
     const int ne = nev < m ? nev : m;
     const bool have_prev = ne == hint_ne;
-    ritz_values<BT>(sa, sb, m, ne, have_prev ? s_hint : nullptr, s_lam, s_lo, s_hi, s_first, &s_flag);
+    ritz_values<BT>(sa, sb, m, ne, have_prev ? s_hint : nullptr, s_lam, s_lo, s_hi, s_first, &s_flag, points);
     // the vectors are formed only once no Ritz value moved by more than tol
     // max(1, |lam|) since the previous check
     if (threadIdx.x == 0) s_full = (last || have_prev) ? 1 : 0;
@@ -124,16 +126,10 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
     do {
       const int j = m;
       // v_j = w / beta; y = H v_j; alpha_j = Re <v_j, y>
-      T v[R];
-      double yr[R], yi[R];
+      T v[R], y[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        set1(v[r], re1(w[r]) * sc, im1(w[r]) * sc);
-        h.apply(r, a.col, a.val, xs, &yr[r], &yi[r]);
-        yr[r] *= sc;
-        yi[r] *= sc;
-      }
-      const double al = b.product(v, yr, yi);
+      for (int r = 0; r < R; ++r) set1(v[r], re1(w[r]) * sc, im1(w[r]) * sc);
+      const double al = b.product(h, a.col, a.val, xs, sc, v, y);
       b.store(j, v);
       // the three-term update first (the big cancellation is then done before
       // any Gram-Schmidt coefficient is formed), then full reorthogonalization
@@ -141,7 +137,9 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
       // |w|^2 (always with dgks off)
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        set1(w[r], yr[r] - al * re1(v[r]) - bprev * re1(vp[r]), yi[r] - al * im1(v[r]) - bprev * im1(vp[r]));
+        w[r] = y[r];
+        add_scaled(w[r], -al, v[r]);
+        add_scaled(w[r], -bprev, vp[r]);
         vp[r] = v[r];
       }
       double p1, pw = 0.0;
@@ -151,7 +149,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
         if (it == 0) pw = before;
         p = 0.0;
 #pragma unroll
-        for (int r = 0; r < R; ++r) p += re1(w[r]) * re1(w[r]) + im1(w[r]) * im1(w[r]);
+        for (int r = 0; r < R; ++r) p = add_re(p, w[r], w[r]);
         publish();
         p1 = b.row_sum(p, 1);
         if (it == 1 || (a.dgks && !(p1 < 0.5 * pw))) break;
@@ -178,7 +176,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) 
     b.combine(m, Y + (size_t)k * L, x);
     p = 0.0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) p += re1(x[r]) * re1(x[r]) + im1(x[r]) * im1(x[r]);
+    for (int r = 0; r < R; ++r) p = add_re(p, x[r], x[r]);
     const double nn = sqrt(b.row_sum(p, 1));
 #pragma unroll
     for (int r = 0; r < R; ++r)

@@ -2060,7 +2060,8 @@ int eigen_flat_chain(const KrylovBatch& kb, int c, int nev, double tol, int max_
 
 namespace {
 
-// Compute units of the current device (one device per process).
+// Compute units of a GPU of this machine (its GPUs are alike; only launch shapes
+// depend on it).
 int device_cus() {
   static const int n = [] {
     int v = 0;
@@ -2089,8 +2090,8 @@ __global__ __launch_bounds__(64) void pure_start_kernel(const int64_t* row_base,
 // Groups of waves per chain of a launch of nb chains: as many as the chip's two
 // waves per SIMD hold for all chains at once (a chain's steps are a dependent
 // sequence, so its waves shorten it; past that they only add barriers), at most
-// lanczos_lds_waves.  Measured, 60-row chains of 60 steps: 873 chains in 2 groups
-// 0.20 ms, in 1 group 0.24 ms; 18432 chains in 1 group 2.45 ms.
+// lanczos_lds_waves.  No bit depends on it.  Measured, 60-row real chains of 60 steps:
+// 873 chains in 2 groups 0.16 ms; 18000 chains in 2 groups 2.6 ms, in 1 group 2.2 ms.
 int reg_groups(unsigned nb, int64_t nmax) {
   const int64_t nq = std::min<int64_t>((nmax + 63) / 64, 4);
   int groups = 4;
@@ -2256,16 +2257,15 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
       (kb.h_n[c] <= lim && dense_eigen_bytes(kb.h_n[c], nev) <= (size_t)150 * 1024 ? dense : rest).push_back(c);
     order.swap(rest);
   }
-  // chains of up to kEigenRegMaxN rows on the register kernels (while no launch
-  // shape is set by hand), by class; beside larger chains, and with a CU for
-  // every chain, all stay in the larger ones' launch, which lasts longer anyway
+  // chains of up to kEigenRegMaxN rows on the register kernels, by class: which
+  // solver a chain gets follows from its own size, whatever else the batch holds
   std::vector<int32_t> reg[kRegClasses];
-  if (g_tuning.eigen_bt == 0) {
+  {
     std::vector<int32_t> rest;
     size_t n_reg = 0;
     for (int32_t c : order) {
       const int64_t n = kb.h_n[c];
-      bool fits = n <= kEigenRegMaxN && n > g_tuning.eigen_wave_max_n;
+      bool fits = n <= kEigenRegMaxN;
       if (fits) {
         EigenArgs t{};
         t.nev = nev;
@@ -2280,12 +2280,8 @@ int run_eigen(const KrylovBatch& kb, int nev, double tol, int max_steps, uint64_
         rest.push_back(c);
       }
     }
-    if (rest.empty() || order.size() > (size_t)device_cus()) {
-      merge_reg_classes(reg, n_reg);
-      order.swap(rest);
-    } else {
-      for (auto& l : reg) l.clear();
-    }
+    merge_reg_classes(reg, n_reg);
+    order.swap(rest);
   }
   std::vector<int64_t> voff(C + 1, 0);
   int64_t R = 0;
@@ -2686,8 +2682,9 @@ extern "C" int imped_lanczos_noalloc(const int64_t* rowptr, const int32_t* col, 
     a.kout = kout;
     a.status = status;
     const size_t shm = reorth ? (size_t)(K + 2) * sizeof(double2) : 0;
-    // the size buckets of run_lanczos, so a chain gets the same kernel (and
-    // the same arithmetic) as through imped_batch_lanczos
+    // the size buckets of run_lanczos; on the register kernels always the complex
+    // instance, whose bits for a real chain are those of the real one: a chain gets
+    // the same bits as through imped_batch_lanczos
     if (reorth && g_tuning.lanczos_lds && lanczos_reg_fits(n, K)) {
       a.nmax = (int)n;
       launch_lanczos_reg(a, 1, s);

@@ -18,8 +18,14 @@
 // own vectors and the update reads them as LDS broadcasts.  With G > 1 the
 // groups' updates meet in LDS (one more barrier).
 //
-// The order of every sum depends on (NQ, G, R) only, not on where a vector
-// sits.
+// The order of every sum is a function of the chain alone: a sum over the basis
+// vectors is formed in kRegParts parts (index mod kRegParts, each in order), of which a
+// group holds kRegParts / G, and added as (p0 + p2) + (p1 + p3); a row of H in
+// kRegRowParts likewise; sums over the rows go by lane, row block and wave, and blocks
+// past the chain's end add zeros.  So NQ, G, R, the element type (for a real or
+// imaginary start vector), the place of a vector, and with them the other chains of a
+// launch, change no bit of a chain's result: its eigenvectors seed plain recurrences
+// whose unconverged part amplifies last bits, and a model must not depend on its batch.
 #pragma once
 
 #include "common.h"
@@ -52,6 +58,8 @@ struct LanczosArgs {
 // Chains of up to this many rows run on the register kernels.
 constexpr int64_t kRegMaxN = 1024;
 constexpr int kRegLds = 160 * 1024;  // LDS of a CU
+constexpr int kRegParts = 4;         // parts of a sum over the basis: the largest number of groups
+constexpr int kRegRowParts = 2;      // parts of a row's sum
 
 // Whether an n-row chain of K steps runs there (its coefficients fit the LDS).
 bool lanczos_reg_fits(int64_t n, int K);

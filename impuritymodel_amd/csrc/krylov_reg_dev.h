@@ -17,6 +17,28 @@ __device__ __forceinline__ double im1(double2 x) { return x.y; }
 __device__ __forceinline__ void set1(double& t, double r, double) { t = r; }
 __device__ __forceinline__ void set1(double2& t, double r, double i) { t = make_double2(r, i); }
 
+// Sums of products, every one an explicit fma in a fixed order, so that the bits do
+// not depend on what the compiler contracts in an instance, and a real vector has the
+// bits it has as a complex one with zero imaginary parts (or, times i, zero real
+// parts): the terms with those parts are +-0.
+// s + Re conj(a) b
+__device__ __forceinline__ double add_re(double s, double a, double b) { return fma(a, b, s); }
+__device__ __forceinline__ double add_re(double s, double2 a, double2 b) { return fma(a.y, b.y, fma(a.x, b.x, s)); }
+// s + a b
+__device__ __forceinline__ void add_mul(double& s, double a, double b) { s = fma(a, b, s); }
+__device__ __forceinline__ void add_mul(double2& s, double2 a, double2 b) {
+  s.x = fma(-a.y, b.y, fma(a.x, b.x, s.x));
+  s.y = fma(a.y, b.x, fma(a.x, b.y, s.y));
+}
+// s + c a, real c
+__device__ __forceinline__ void add_scaled(double& s, double c, double a) { s = fma(c, a, s); }
+__device__ __forceinline__ void add_scaled(double2& s, double c, double2 a) {
+  s.x = fma(c, a.x, s.x);
+  s.y = fma(c, a.y, s.y);
+}
+__device__ __forceinline__ double sum1(double a, double b) { return a + b; }
+__device__ __forceinline__ double2 sum1(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>): every
 // index of a register array is then a constant, so the array stays in
 // registers.
@@ -63,12 +85,28 @@ __device__ __forceinline__ double wave_sum8(const double (&x)[8], bool odd8) {
   return r;
 }
 
+// Every value summed over the wave, by the same tree of lanes for N = 1 and 2.
+template <int N>
+__device__ __forceinline__ void wave_sums(double (&x)[N]) {
+  double r = halve_swap<32>(x[0], x[N - 1]);  // value k in half k of the wave (N = 2)
+  r = halve_swap<16>(r, r);
+  r += dpp_move<0x128, 0xF>(r);  // row_ror:8
+  r += dpp_move<0x141, 0xF>(r);  // row_half_mirror
+  r += dpp_move<0x4E, 0xF>(r);   // quad_perm [2,3,0,1]
+  r += dpp_move<0xB1, 0xF>(r);   // quad_perm [1,0,3,2]
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    x[k] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(r), 64 / N * k),
+                            __builtin_amdgcn_readlane(__double2loint(r), 64 / N * k));
+}
+
 // Vectors of the basis in registers and entries of each row of H beside them:
-// the most that the 256 registers of a thread hold without spilling.
+// the most that the 256 registers of a thread hold without spilling (one wave alone
+// also keeps all parts of the sums).
 template <int W, int R, class T>
 constexpr int reg_slots() {
-  if (reg_real_v<T>) return R == 1 ? 72 : R == 2 ? 24 : 8;
-  return R == 1 ? (W == 1 ? 36 : 32) : R == 2 ? 8 : 4;
+  if (reg_real_v<T>) return R == 1 ? (W == 1 ? 56 : 72) : R == 2 ? 24 : 8;
+  return R == 1 ? 32 : R == 2 ? 8 : 4;
 }
 template <int R, class T>
 constexpr int reg_row_entries() {
@@ -82,6 +120,9 @@ struct RegBasis {
   static constexpr int S = reg_slots<W, R, T>();    // register slots per thread
   static constexpr int B = reg_real_v<T> ? 8 : 4;   // vectors per reduction of eight values
   static constexpr int D = reg_real_v<T> ? 1 : 2;   // doubles per element
+  static constexpr int F = kRegParts / G;           // parts of every sum that a group forms
+  static_assert(G > 1 || W == 1, "one group of several waves: product has no case for it");
+  static_assert(S % kRegParts == 0 && B % kRegParts == 0, "a part's vectors must not depend on where they sit");
 
   double vr[S][R], vi[reg_real_v<T> ? 1 : S][R];  // the register slots
   int lane, wave, q, g;
@@ -94,14 +135,16 @@ struct RegBasis {
   double* dotp;  // LDS [NQ][lcap * D * G]: dots of wave q's rows, by group and local index
   double* cw;    // LDS [W][lcap * D]: this wave's coefficients
   T* upd;       // LDS [G][NQ*64*R]: the groups' updates, and parts of H v (G > 1)
-  double* red;  // LDS [3][W]
+  double* red;  // LDS [2][W] and [kRegRowParts][NQ]
   int lcap;     // local vectors per group, a multiple of B
+
+  static constexpr int kRed = 2 * W + kRegRowParts * NQ;  // (even)
 
   // doubles of LDS before the vectors for chains of K steps
   static __host__ __device__ int lcap_for(int K) { return ((K + G - 1) / G + B - 1) / B * B; }
   static __host__ __device__ size_t fixed_doubles(int K) {
     const size_t lc = (size_t)lcap_for(K) * D;
-    return (size_t)NQ * G * lc + (NQ > 1 ? (size_t)W * lc : 0) + (G > 1 ? (size_t)G * NQ * 64 * R * D : 0) + 3 * W + (W & 1);
+    return (size_t)NQ * G * lc + (NQ > 1 ? (size_t)W * lc : 0) + (G > 1 ? (size_t)G * NQ * 64 * R * D : 0) + kRed;
   }
 
   __device__ __forceinline__ void init(int n_, int K, int kl_, double* lds, T* vstore) {
@@ -119,7 +162,7 @@ struct RegBasis {
     upd = reinterpret_cast<T*>(p);
     p += G > 1 ? (size_t)G * NQ * 64 * R * D : 0;
     red = p;
-    p += 3 * W + (W & 1);
+    p += kRed;
     vl = reinterpret_cast<T*>(p);
     vg = vstore;
 #pragma unroll
@@ -198,19 +241,15 @@ struct RegBasis {
   }
 
   // dots of B vectors with w over this wave's rows, into the dots array
-  template <class F>
-  __device__ __forceinline__ void dot_batch(int li, int nl, const T (&w)[R], F&& x) {
+  template <class X>
+  __device__ __forceinline__ void dot_batch(int li, int nl, const T (&w)[R], X&& x) {
     double p[8];
     static_for<B>([&](auto s) __attribute__((always_inline)) {
       double px = 0.0, py = 0.0;
       static_for<R>([&](auto r) __attribute__((always_inline)) {
         const T a = x(s, r);
-        px += re1(a) * re1(w[r]);
-        if constexpr (!reg_real_v<T>) {
-          px += im1(a) * im1(w[r]);
-          py += re1(a) * im1(w[r]);
-          py -= im1(a) * re1(w[r]);
-        }
+        px = add_re(px, a, w[r]);
+        if constexpr (!reg_real_v<T>) py = fma(-im1(a), re1(w[r]), fma(re1(a), im1(w[r]), py));
       });
       p[s * D] = px;
       if constexpr (!reg_real_v<T>) p[s * D + 1] = py;
@@ -221,28 +260,41 @@ struct RegBasis {
     if ((lane & 7) == 0) dst[(size_t)li * D + (lane >> 3)] = d;
   }
 
-  template <class F>
-  __device__ __forceinline__ void upd_batch(int li, T (&u0)[R], T (&u1)[R], F&& x) {
+  template <class X>
+  __device__ __forceinline__ void upd_batch(int li, T (&u)[F][R], X&& x) {
     const T* c = reinterpret_cast<const T*>(cw) + li;
     static_for<B>([&](auto s) __attribute__((always_inline)) {
       const T cs = c[s];
-      static_for<R>([&](auto r) __attribute__((always_inline)) {
-        const T a = x(s, r);
-        T& u = s & 1 ? u1[r] : u0[r];
-        if constexpr (reg_real_v<T>) {
-          u += a * cs;
-        } else {
-          u.x += a.x * cs.x;
-          u.x -= a.y * cs.y;
-          u.y += a.x * cs.y;
-          u.y += a.y * cs.x;
-        }
-      });
+      static_for<R>([&](auto r) __attribute__((always_inline)) { add_mul(u[s % F][r], x(s, r), cs); });
     });
   }
 
+  // The parts of one group, and of the groups, added up: (p0 + p2) + (p1 + p3)
+  // whatever the number of groups (group g has parts g, g + G, ...).
+  template <class U>
+  static __device__ __forceinline__ U own_parts(const U (&p)[F]) {
+    if constexpr (F == 4)
+      return sum1(sum1(p[0], p[2]), sum1(p[1], p[3]));
+    else if constexpr (F == 2)
+      return sum1(p[0], p[1]);
+    else
+      return p[0];
+  }
+  __device__ __forceinline__ void put_part(int r, const T& t) const {
+    upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane] = t;
+  }
+  __device__ __forceinline__ T get_part(int k, int r) const {
+    return upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
+  }
+  __device__ __forceinline__ T all_parts(int r) const {
+    if constexpr (G == 4)
+      return sum1(sum1(get_part(0, r), get_part(2, r)), sum1(get_part(1, r), get_part(3, r)));
+    else
+      return sum1(get_part(0, r), get_part(1, r));
+  }
+
   // sum of x over the chain's rows (x: this thread's part; the same in every
-  // group), slot k of three used in turn: one barrier
+  // group), slot k of red (0: pass): one barrier
   __device__ __forceinline__ double row_sum(double x, int k) {
     x = wave_sum(x);
     if constexpr (W == 1) return x;
@@ -258,32 +310,45 @@ struct RegBasis {
     return t;
   }
 
-  // (yr, yi) <- the groups' parts of H v summed; returns Re <v, H v>.  One
-  // barrier: the parts and each wave's share of the product go to LDS together.
-  __device__ __forceinline__ double product(const T (&v)[R], double (&yr)[R], double (&yi)[R]) {
-    double p = 0.0;
+  // y = sc H x from RegRows (x in LDS), and Re <v, y>.  One barrier: the groups'
+  // parts of y and each wave's parts of the product go to LDS together.
+  template <class H>
+  __device__ __forceinline__ double product(const H& h, const int32_t* col, const double2* val, const T* x, double sc,
+                                            const T (&v)[R], T (&y)[R]) {
+    double p[H::F];
 #pragma unroll
-    for (int r = 0; r < R; ++r) p += re1(v[r]) * yr[r] + im1(v[r]) * yi[r];
-    if constexpr (G == 1) return row_sum(p, 2);
-    p = wave_sum(p);
-    if (lane == 0) red[2 * W + wave] = p;
-#pragma unroll
-    for (int r = 0; r < R; ++r) set1(upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane], yr[r], yi[r]);
-    __syncthreads();
-    p = 0.0;
-#pragma unroll
-    for (int k = 0; k < W; ++k) p += red[2 * W + k];
+    for (int f = 0; f < H::F; ++f) p[f] = 0.0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      yr[r] = yi[r] = 0.0;
+      T part[H::F];
+      h.apply(r, col, val, x, part);
 #pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const T t = upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
-        yr[r] += re1(t);
-        yi[r] += im1(t);
+      for (int f = 0; f < H::F; ++f) {
+        set1(part[f], re1(part[f]) * sc, im1(part[f]) * sc);
+        p[f] = add_re(p[f], v[r], part[f]);
       }
+      y[r] = part[0];
+      if constexpr (H::F == 2) y[r] = sum1(part[0], part[1]);
     }
-    return p;
+    wave_sums(p);
+    if constexpr (W == 1) return p[0] + p[1];
+    double* rp = red + 2 * W;
+    if (g < kRegRowParts) {
+      if (lane == 0) rp[g * NQ + q] = p[0];
+#pragma unroll
+      for (int r = 0; r < R; ++r) put_part(r, y[r]);
+    }
+    __syncthreads();
+    double t[kRegRowParts];
+#pragma unroll
+    for (int k = 0; k < kRegRowParts; ++k) {
+      t[k] = rp[k * NQ];
+#pragma unroll
+      for (int i = 1; i < NQ; ++i) t[k] += rp[k * NQ + i];
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) y[r] = sum1(get_part(0, r), get_part(1, r));
+    return t[0] + t[1];
   }
 
   // One classical Gram-Schmidt pass of w against vectors 0..m-1; *pw receives
@@ -292,7 +357,7 @@ struct RegBasis {
     const int nl = __builtin_amdgcn_readfirstlane((m - g + G - 1) / G);  // this group's vectors
     double p = 0.0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) p += re1(w[r]) * re1(w[r]) + im1(w[r]) * im1(w[r]);
+    for (int r = 0; r < R; ++r) p = add_re(p, w[r], w[r]);
     p = wave_sum(p);
     if constexpr (NQ > 1) {
       if (lane == 0) red[wave] = p;
@@ -329,97 +394,99 @@ struct RegBasis {
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
     *pw = p;
-    T u0[R], u1[R];
+    T u[F][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      set1(u0[r], 0.0, 0.0);
-      set1(u1[r], 0.0, 0.0);
-    }
+    for (int k = 0; k < F * R; ++k) set1(u[k / R][k % R], 0.0, 0.0);
     static_for<S / B>([&](auto bc) __attribute__((always_inline)) {
       constexpr int b = bc * B;
-      if (b < nl) upd_batch(b, u0, u1, [&](auto s, auto r) __attribute__((always_inline)) { return slot<b + s, r>(); });
+      if (b < nl) upd_batch(b, u, [&](auto s, auto r) __attribute__((always_inline)) { return slot<b + s, r>(); });
     });
     for (int li = S; li < n1; li += B) {
       T x[B][R];
       fetch_lds(li, n1, x);
-      upd_batch(li, u0, u1, [&](auto s, auto r) __attribute__((always_inline)) { return x[s][r]; });
+      upd_batch(li, u, [&](auto s, auto r) __attribute__((always_inline)) { return x[s][r]; });
     }
     for (int li = S + kl; li < nl; li += B) {
       T x[B][R];
       fetch_mem(li, nl, x);
-      upd_batch(li, u0, u1, [&](auto s, auto r) __attribute__((always_inline)) { return x[s][r]; });
+      upd_batch(li, u, [&](auto s, auto r) __attribute__((always_inline)) { return x[s][r]; });
     }
-    if constexpr (G == 1) {
+    T d[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (on[r]) set1(w[r], re1(w[r]) - (re1(u0[r]) + re1(u1[r])), im1(w[r]) - (im1(u0[r]) + im1(u1[r])));
-    } else {
+    for (int r = 0; r < R; ++r) d[r] = gather(u, r);
+    if constexpr (G > 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        set1(upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane], re1(u0[r]) + re1(u1[r]), im1(u0[r]) + im1(u1[r]));
+      for (int r = 0; r < R; ++r) put_part(r, d[r]);
       __syncthreads();
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        double ux = 0.0, uy = 0.0;
-#pragma unroll
-        for (int k = 0; k < G; ++k) {
-          const T t = upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
-          ux += re1(t);
-          uy += im1(t);
-        }
-        if (on[r]) set1(w[r], re1(w[r]) - ux, im1(w[r]) - uy);
-      }
+      for (int r = 0; r < R; ++r) d[r] = all_parts(r);
     }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (on[r]) set1(w[r], re1(w[r]) - re1(d[r]), im1(w[r]) - im1(d[r]));
+  }
+  static __device__ __forceinline__ T gather(const T (&u)[F][R], int r) {
+    T p[F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) p[f] = u[f][r];
+    return own_parts(p);
   }
 
   // x = sum over l < m of y[l] v_l (real y; the same sum in every group)
   __device__ __forceinline__ void combine(int m, const double* y, T (&out)[R]) {
     const int nl = __builtin_amdgcn_readfirstlane((m - g + G - 1) / G);
-    double ur[R], ui[R];
+    T u[F][R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) ur[r] = ui[r] = 0.0;
-    auto add = [&](double c, int r, const T& t) __attribute__((always_inline)) {
-      ur[r] += c * re1(t);
-      if constexpr (!reg_real_v<T>) ui[r] += c * im1(t);
-    };
+    for (int k = 0; k < F * R; ++k) set1(u[k / R][k % R], 0.0, 0.0);
     static_for<S>([&](auto s) __attribute__((always_inline)) {
       if (s < nl)
-        static_for<R>([&](auto r) __attribute__((always_inline)) { add(y[s * G + g], r, slot<s, r>()); });
+        static_for<R>([&](auto r) __attribute__((always_inline)) {
+          add_scaled(u[s % F][r], y[s * G + g], slot<s, r>());
+        });
     });
     const int n1 = nl < S + kl ? nl : S + kl;
-    for (int li = S; li < n1; ++li)
+    for (int li = S; li < n1; li += F)
 #pragma unroll
-      for (int r = 0; r < R; ++r) add(y[li * G + g], r, vl[(size_t)((li - S) * G + g) * n + row[r]]);
-#pragma unroll 4
-    for (int li = S + kl; li < nl; ++li)
+      for (int f = 0; f < F; ++f)
+        if (li + f < n1)
 #pragma unroll
-      for (int r = 0; r < R; ++r) add(y[li * G + g], r, vg[(size_t)(li * G + g) * n + row[r]]);
+          for (int r = 0; r < R; ++r)
+            add_scaled(u[f][r], y[(li + f) * G + g], vl[(size_t)((li + f - S) * G + g) * n + row[r]]);
+#pragma unroll 4 / F
+    for (int li = S + kl; li < nl; li += F)
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        if (li + f < nl)
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+            add_scaled(u[f][r], y[(li + f) * G + g], vg[(size_t)((li + f) * G + g) * n + row[r]]);
+    T d[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) d[r] = gather(u, r);
     if constexpr (G > 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) set1(upd[((size_t)g * R + r) * NQ * 64 + q * 64 + lane], ur[r], ui[r]);
+      for (int r = 0; r < R; ++r) put_part(r, d[r]);
       __syncthreads();
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        ur[r] = ui[r] = 0.0;
-#pragma unroll
-        for (int k = 0; k < G; ++k) {
-          const T t = upd[((size_t)k * R + r) * NQ * 64 + q * 64 + lane];
-          ur[r] += re1(t);
-          ui[r] += im1(t);
-        }
-      }
+      for (int r = 0; r < R; ++r) d[r] = all_parts(r);
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) set1(out[r], on[r] ? ur[r] : 0.0, on[r] ? ui[r] : 0.0);
+    for (int r = 0; r < R; ++r) set1(out[r], on[r] ? re1(d[r]) : 0.0, on[r] ? im1(d[r]) : 0.0);
   }
 };
 
-// The rows of H of one thread: group g takes entries g, g + G, ... of each row,
-// up to HR of them in registers, the rest read from memory (the groups'
-// products of a row meet in RegBasis::product).
+// The rows of H of one thread: entry e of a row counts to part e % kRegRowParts of its
+// sum (the parts meet in RegBasis::product).  Group g takes part g % kRegRowParts, a
+// single group both; up to HR of its entries are in registers, the rest read from
+// memory.  (Four parts would divide the rows over four groups, but one group alone
+// then spills: 18432 complex chains of 60 rows 2.7 ms, with two parts 2.5 ms; two
+// chains of 100 rows in four groups each 406 and 403 us.)
 template <int W, int G, int R, class T>
 struct RegRows {
   static constexpr int HR = reg_row_entries<R, T>();
+  static constexpr int N = G < kRegRowParts ? G : kRegRowParts;  // groups that share a row
+  static constexpr int F = kRegRowParts / N;                     // parts that each forms
+  static_assert(HR % 2 == 0, "an entry's part must not depend on where it sits");
   T h[R][HR ? HR : 1];
   int c[R][HR ? HR : 1];
   int cnt_wave[R];
@@ -427,6 +494,7 @@ struct RegRows {
 
   __device__ __forceinline__ void load(const int64_t* rowptr, const int32_t* col, const double2* val, int g,
                                        const int (&row)[R], const bool (&on)[R]) {
+    g %= N;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       int cnt = 0;
@@ -435,63 +503,52 @@ struct RegRows {
       if (on[r]) {
         e0 = rowptr[row[r]] + g;
         end[r] = rowptr[row[r] + 1];
-        const int64_t mine = end[r] > e0 ? (end[r] - e0 + G - 1) / G : 0;
+        const int64_t mine = end[r] > e0 ? (end[r] - e0 + N - 1) / N : 0;
         cnt = (int)(mine < HR ? mine : HR);
-        rest[r] = e0 + (int64_t)cnt * G;
+        rest[r] = e0 + (int64_t)cnt * N;
       }
 #pragma unroll
       for (int k = 0; k < HR; ++k) {
         set1(h[r][k], 0.0, 0.0);
         c[r][k] = 0;
         if (k < cnt) {
-          const double2 t = val[e0 + (int64_t)k * G];
+          const double2 t = val[e0 + (int64_t)k * N];
           set1(h[r][k], t.x, t.y);
-          c[r][k] = col[e0 + (int64_t)k * G];
+          c[r][k] = col[e0 + (int64_t)k * N];
         }
       }
       cnt_wave[r] = wave_max_int(cnt);
     }
   }
 
-  // this group's part of row r of H x (x in LDS)
-  __device__ __forceinline__ void apply(int r, const int32_t* col, const double2* val, const T* x, double* yr,
-                                        double* yi) const {
-    double ax = 0.0, ay = 0.0, bx = 0.0, by = 0.0;
-    auto add = [](double& sx, double& sy, const T& a, const T& b) {
-      sx += re1(a) * re1(b);
-      if constexpr (!reg_real_v<T>) {
-        sx -= im1(a) * im1(b);
-        sy += re1(a) * im1(b);
-        sy += im1(a) * re1(b);
-      }
-    };
+  // this group's parts of row r of H x (x in LDS)
+  __device__ __forceinline__ void apply(int r, const int32_t* col, const double2* val, const T* x,
+                                        T (&part)[F]) const {
+#pragma unroll
+    for (int f = 0; f < F; ++f) set1(part[f], 0.0, 0.0);
 #pragma unroll
     for (int k0 = 0; k0 < HR; k0 += 4)
       if (k0 < cnt_wave[r]) {
         T t[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) t[u] = x[c[r][k0 + u]];
-        add(ax, ay, h[r][k0], t[0]);
-        add(bx, by, h[r][k0 + 1], t[1]);
-        add(ax, ay, h[r][k0 + 2], t[2]);
-        add(bx, by, h[r][k0 + 3], t[3]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) add_mul(part[u % F], h[r][k0 + u], t[u]);
       }
     // four entries per round trip (indices past the row clamped, their products skipped)
-    for (int64_t e = rest[r]; e < end[r]; e += 4 * G) {
+    for (int64_t e = rest[r]; e < end[r]; e += 4 * N) {
       T hh[4], t[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int64_t k = e + u * G < end[r] ? e + u * G : end[r] - 1;
+        const int64_t k = e + u * N < end[r] ? e + u * N : end[r] - 1;
         const double2 z = val[k];
         set1(hh[u], z.x, z.y);
         t[u] = x[col[k]];
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (e + u * G < end[r]) add(ax, ay, hh[u], t[u]);
+        if (e + u * N < end[r]) add_mul(part[u % F], hh[u], t[u]);
     }
-    *yr = ax + bx;
-    *yi = ay + by;
   }
 };
 

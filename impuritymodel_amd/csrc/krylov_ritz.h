@@ -186,9 +186,10 @@ struct EigenArgs {
 };
 
 // Lowest nev eigenvalues of the symmetric tridiagonal (a, b) of size m by
-// multisection: the workgroup splits into nev groups; each evaluates Sturm
-// counts at G interior points of its interval per round and keeps the
-// sub-interval where the count crosses k, shrinking it G+1 times per round.
+// multisection: the workgroup's first `points` threads split into nev groups; each
+// evaluates Sturm counts at G interior points of its interval per round and keeps
+// the sub-interval where the count crosses k, shrinking it G+1 times per round.
+// The values' last bits depend on `points` alone, not on BT.
 // hint (or null): the same eigenvalues of a leading block of (a, b).  By
 // Cauchy interlacing they bound the new ones from above, so a first round of
 // points hint - scale 10^(-16 r / (G-2)) (r < G-1) and hint + 1e-14 scale
@@ -197,7 +198,7 @@ struct EigenArgs {
 // hint does not bracket it).
 template <int BT>
 __device__ __forceinline__ void ritz_values(const double* a, const double* b, int m, int nev, const double* hint, double* s_lam,
-                            double* s_lo, double* s_hi, int* s_first, int* s_flag) {
+                            double* s_lo, double* s_hi, int* s_first, int* s_flag, int points = BT) {
   __shared__ double s_part[3][BT / 64];
   __shared__ double s_bounds[3];
   {
@@ -231,7 +232,7 @@ __device__ __forceinline__ void ritz_values(const double* a, const double* b, in
     }
   }
   __syncthreads();
-  const int G = BT / nev;
+  const int G = points / nev;
   const int g = threadIdx.x / G, r = threadIdx.x % G;
   const double scale = s_bounds[2];
   if ((int)threadIdx.x < nev) {

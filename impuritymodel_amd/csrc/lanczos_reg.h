@@ -73,22 +73,18 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs
   int kdone = K, status = IMPED_OK;
   for (int j = 0;; ++j) {
     // v_j = w / beta; y = H v_j; alpha_j = Re <v_j, y>
-    T v[R];
-    double yr[R], yi[R];
+    T v[R], y[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      set1(v[r], re1(w[r]) * sc, im1(w[r]) * sc);
-      h.apply(r, a.col, a.val, xs, &yr[r], &yi[r]);
-      yr[r] *= sc;
-      yi[r] *= sc;
-    }
-    const double al = b.product(v, yr, yi);
+    for (int r = 0; r < R; ++r) set1(v[r], re1(w[r]) * sc, im1(w[r]) * sc);
+    const double al = b.product(h, a.col, a.val, xs, sc, v, y);
     if (threadIdx.x == 0) alpha[j] = al;
     if (j + 1 == K) break;
     b.store(j, v);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      set1(w[r], yr[r] - al * re1(v[r]) - beta_j * re1(vp[r]), yi[r] - al * im1(v[r]) - beta_j * im1(vp[r]));
+      w[r] = y[r];
+      add_scaled(w[r], -al, v[r]);
+      add_scaled(w[r], -beta_j, vp[r]);
       vp[r] = v[r];
     }
     // full reorthogonalization against v_0..v_j; a second pass when the
@@ -100,7 +96,7 @@ __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs
       if (it == 0) pw = before;
       p = 0.0;
 #pragma unroll
-      for (int r = 0; r < R; ++r) p += re1(w[r]) * re1(w[r]) + im1(w[r]) * im1(w[r]);
+      for (int r = 0; r < R; ++r) p = add_re(p, w[r], w[r]);
       publish();
       p1 = b.row_sum(p, 1);
       if (it == 1 || !(p1 < 0.5 * pw)) break;

@@ -58,10 +58,12 @@ int imped_timing_query(const char* name, double* total_ms, int64_t* launches);
 
 /* Launch-shape parameters picked per chain-dimension bucket; no reference
  * counterpart.  Names: "lanczos_wave_max_n", "lanczos_wg256_max_n" (Lanczos
- * threads per chain: 64 / 256 / 1024 by size), "eigen_wave_max_n" (eigensolver
- * chains up to this size get one wave), "eigen_bt" (threads per larger
- * eigensolver chain: 256, 512, 1024; 0, the default: 1024 when the launch's
- * largest chain has more than 512 rows, else 512), "eigen_real", "eigen_dgks",
+ * threads per chain: 64 / 256 / 1024 by size), "eigen_wave_max_n" (chains that
+ * the eigensolver keeps in memory, those beyond 512 rows or beyond the LDS, get
+ * one wave up to this size), "eigen_bt" (threads per larger one of them: 256,
+ * 512, 1024; 0, the default: 1024 when the launch's largest chain has more than
+ * 512 rows, else 512; every other chain runs on the register kernels, whatever
+ * these two say), "eigen_real", "eigen_dgks",
  * "eigen_check_every" (Ritz convergence check every this many steps, 12 by
  * default), "eigen_check_start" (no Ritz convergence check before
  * min(this, n/2) steps of an n-row chain, 48 by default; the last step is
@@ -79,8 +81,8 @@ int imped_timing_query(const char* name, double* total_ms, int64_t* launches);
  * CSR; 0: the complex values),
  * "lanczos_graph_steps" (grid-wide Lanczos steps per replayed HIP graph,
  * 0..256; 0 launches every step directly, as does switched-on timing),
- * "eigen_lds_vectors" (cap on the Krylov vectors the eigensolver keeps in
- * LDS; -1 as many as fit, 0 none), "small_sort" (1: key sets of at most
+ * "eigen_lds_vectors" (cap on the Krylov vectors, per group of waves, that the
+ * register eigensolver keeps in LDS; -1 as many as fit, 0 none), "small_sort" (1: key sets of at most
  * 16384 records whose chain, key and position fit 63 bits are sorted by one
  * workgroup; 0: always the digit passes), "mlp_graph" (1: a surrogate
  * prediction's kernels run as one replayed HIP graph, which shortens the
@@ -288,7 +290,8 @@ int imped_batch_lanczos(imped_batch batch, const double* v0, int K, int reorth, 
                         int32_t* kout, int32_t* status);
 
 /* Allocation-free variant of imped_batch_lanczos for one chain: the same
- * Lanczos kernel (plain recurrence, or reorth = 1) on a CSR, start vector and
+ * results, bit for bit below the grid-wide threshold (plain recurrence, or
+ * reorth = 1, complex arithmetic throughout), on a CSR, start vector and
  * outputs that the caller holds in DEVICE memory -- rowptr[n+1] int64, col
  * int32, val complex, v0[n] complex, alpha[K], beta[K], kout[1], status[1] --
  * queued on `stream` (a hipStream_t; NULL = the null stream) without

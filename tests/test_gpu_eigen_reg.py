@@ -69,3 +69,43 @@ def test_eigensolver_reports_missed_tolerance(gpu, n):
     ev, _, steps, ok = b.eigen(3, tol=1e-12, max_steps=8, allow_noconv=True)
     assert not ok and steps[0] == 8
     assert np.all(np.isfinite(ev))
+
+
+@pytest.mark.parametrize("complex_h", [True, False])
+@pytest.mark.parametrize("n", [2, 40, 64, 100, 190, 256, 448])
+def test_eigensolver_does_not_depend_on_the_batch(gpu, complex_h, n):
+    """A chain on the register kernels has the same pairs, bit for bit, alone, among so many chains that
+    the waves per chain change, beside chains whose launch it joins or that other kernels solve, and
+    with the launch shapes of those kernels set by hand."""
+    from impuritymodel_amd import engine
+
+    h = _chain(n, complex_h, -700.0)
+    small, empty = _chain(50, complex_h, 0.0), np.zeros((0, 0))
+    batches = {"alone": [], "empty": [empty], "same": [_chain(n, complex_h, 3.0)], "joined": [_chain(500, complex_h, 0.0)],
+               "memory": [_chain(600, complex_h, 0.0)], "wide": [_chain(1500, complex_h, 0.0), small],
+               "many": [small] * 600, "most": [_chain(70, complex_h, 1.0)] * 2200}
+    want = None
+
+    def check(rest, name):
+        nonlocal want
+        b = _batch([h] + rest)
+        ev, vecs, steps, ok = b.eigen(3, tol=1e-12)
+        got = (ev[0], vecs[:3 * n], steps[0])
+        want = want or got
+        assert ok
+        assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1]), name
+        assert got[2] == want[2], name
+
+    for name, rest in batches.items():
+        check(rest, name)
+    try:
+        for knob, value in (("eigen_bt", 256), ("eigen_bt", 512), ("eigen_bt", 1024), ("eigen_wave_max_n", 1024),
+                            ("lanczos_lds_waves", 1), ("eigen_lds_vectors", 0)):
+            engine.set_tuning(knob, value)
+            check([], knob)
+            check(batches["wide"], knob)
+            engine.set_tuning(knob, {"eigen_bt": 0, "eigen_wave_max_n": 0, "lanczos_lds_waves": 4,
+                                     "eigen_lds_vectors": -1}[knob])
+    finally:
+        for knob, value in (("eigen_bt", 0), ("eigen_wave_max_n", 0), ("lanczos_lds_waves", 4), ("eigen_lds_vectors", -1)):
+            engine.set_tuning(knob, value)

@@ -47,7 +47,7 @@ def _chain(rng, n, complex_h, start):
     return scipy.sparse.csr_matrix(h.astype(complex)), v / np.linalg.norm(v)
 
 
-def _run(chains, K):
+def _built(chains):
     from impuritymodel_amd.engine import Batch, Ops
 
     b = Batch(Ops([{}], [None], 1), np.zeros(len(chains), np.int32))
@@ -57,7 +57,11 @@ def _run(chains, K):
     b.set_csr([h.shape[0] for h, _ in chains], np.array(rowptr, np.int64),
               np.concatenate([h.indices for h, _ in chains]).astype(np.int32),
               np.concatenate([h.data for h, _ in chains]))
-    return b.lanczos(K, reorth=1, v0=np.concatenate([v for _, v in chains]))
+    return b
+
+
+def _run(chains, K):
+    return _built(chains).lanczos(K, reorth=1, v0=np.concatenate([v for _, v in chains]))
 
 
 @pytest.mark.parametrize("complex_h,start", [(True, "complex"), (False, "complex"), (False, "real"),
@@ -116,3 +120,37 @@ def test_register_lanczos_launch_of_empty_chains_only(gpu, complex_h, n_empty, o
         assert (kout[n_empty:] == 12).all() and not status[n_empty:].any()
         scale = max(1.0, abs(chain[0]).sum(axis=1).max())
         assert np.abs(alpha[n_empty:] - a).max() <= 1e-10 * scale
+
+
+@pytest.mark.parametrize("complex_h,start", [(True, "complex"), (False, "complex"), (False, "real"),
+                                             (False, "imaginary")])
+@pytest.mark.parametrize("n,K", [(40, 40), (64, 64), (100, 100), (150, 80), (225, 150), (300, 90), (600, 60), (900, 40)])
+def test_register_lanczos_does_not_depend_on_the_batch(gpu, complex_h, start, n, K):
+    """The same bits alone, among so many chains that the waves per chain change, beside a chain
+    whose launch it joins, with fewer waves by hand, and, for a real H, in the complex arithmetic
+    that a complex chain in the batch brings."""
+    from impuritymodel_amd import engine
+
+    rng = np.random.default_rng(n)
+    chain = _chain(rng, n, complex_h, start)
+    wide = _chain(rng, n, complex_h, start)  # rows longer than the entries kept in registers
+    dense = scipy.sparse.random(n, n, density=0.3, random_state=rng).tocsr()
+    wide = ((wide[0] + (dense + dense.T)).tocsr(), wide[1])
+    others = {"alone": [], "pair": [_chain(rng, n, complex_h, start)], "larger": [_chain(rng, 1000, complex_h, "real")],
+              "middle": [_chain(rng, 260, complex_h, "complex")], "complex": [_chain(rng, 30, True, "complex")],
+              "many": [_chain(rng, 33, complex_h, start)] * 600, "most": [_chain(rng, 65, complex_h, start)] * 2200}
+    for c in (chain, wide):
+        want = None
+        for name, rest in others.items():
+            alpha, beta, kout, status = _run([c] + rest, K)
+            got = (alpha[0, :kout[0]], beta[0, :kout[0] - 1])
+            assert (kout[0], status[0]) == (min(K, n), 0), name
+            want = want or got
+            assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), name
+        try:
+            for waves in (1, 2):
+                engine.set_tuning("lanczos_lds_waves", waves)
+                alpha, beta, kout, _ = _run([c], K)
+                assert np.array_equal(alpha[0, :kout[0]], want[0]) and np.array_equal(beta[0, :kout[0] - 1], want[1])
+        finally:
+            engine.set_tuning("lanczos_lds_waves", 4)

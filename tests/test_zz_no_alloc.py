@@ -1,8 +1,9 @@
 """imped_lanczos_noalloc (the allocation-free Lanczos entry point) against
 imped_batch_lanczos on the same CSR and start vector.
 
-The two entry points run the same kernel for chains up to the grid-wide
-threshold, so alpha, beta, kout and status must agree bit for bit.  Two calls
+The two entry points sum in the same order for chains up to the grid-wide
+threshold (also where the batch one works in real arithmetic), so alpha, beta,
+kout and status must agree bit for bit.  Two calls
 in a row, the second on a smaller chain, check that the shared scratch array
 carries nothing over; a chain beyond the scratch capacity is refused.
 """
@@ -88,3 +89,20 @@ def test_noalloc_lanczos_refuses_chain_beyond_scratch(gpu):
     # with reorthogonalization the Krylov vectors count too
     rc = lib.imped_lanczos_noalloc(p, p, p, 30_000, p, 200, 1, p, p, p, p, None)
     assert rc == IMPED_ERR_CAPACITY
+
+
+@pytest.mark.parametrize("start", ["real", "imaginary", "complex"])
+@pytest.mark.parametrize("n,K", [(60, 60), (200, 100), (600, 60), (900, 40)])
+def test_noalloc_equals_batch_for_a_real_matrix(gpu, n, K, start):
+    # the batch entry point takes real arithmetic for a real H and a real or imaginary start vector
+    rng = np.random.default_rng(n)
+    a = scipy.sparse.random(n, n, density=6.0 / n, random_state=rng, data_rvs=lambda k: rng.standard_normal(k))
+    h = (a + a.T + scipy.sparse.diags(rng.standard_normal(n) * 3)).tocsr().astype(complex)
+    h.sort_indices()
+    v0 = rng.standard_normal(n) + (1j * rng.standard_normal(n) if start == "complex" else 0.0)
+    v0 = v0 / np.linalg.norm(v0) * (1j if start == "imaginary" else 1.0)
+    a_ref, b_ref, k_ref, s_ref = _batch(h, v0, K, 1)
+    got_a, got_b, ks = _noalloc(h, v0, K, 1)
+    kk = min(K, n)
+    assert (int(ks[0]), int(ks[1])) == (k_ref, s_ref) == (kk, 0)
+    assert np.array_equal(got_a[:kk], a_ref[:kk]) and np.array_equal(got_b[:kk - 1], b_ref[:kk - 1])
