@@ -6,8 +6,10 @@ chosen per chain-dimension bucket:
 * ``lanczos_wave_max_n``: chains up to this size run the Lanczos recurrence
   in one wave (shuffle reductions, no barriers); larger ones get 256 or 1024
   threads;
-* ``eigen_bt``, ``eigen_check_every``, ``eigen_wave_max_n``: threads per
-  eigensolver chain, Ritz-check interval, one-wave bucket;
+* ``eigen_bt``, ``eigen_wave_max_n``: threads per eigensolver chain and the
+  one-wave bucket, of chains whose Krylov basis is in memory (chains on the
+  register kernels, up to 512 rows, have their own rule);
+* ``eigen_check_every``: Ritz-check interval;
 * ``spmv_lpr``: lanes per CSR row of the grid-wide SpMV (sectors above
   ``flat_min_n``).
 
@@ -41,7 +43,7 @@ DEFAULTS = {
 
 CANDIDATES = {
     "lanczos_wave_max_n": [512, 1024, 4096, 16384],
-    "eigen_bt": [256, 512, 1024],
+    "eigen_bt": [0, 256, 512, 1024],  # 0, by size, first: kept where the times are equal
     "eigen_check_every": [4, 8, 12, 16],
     "eigen_wave_max_n": [0, 256, 1024],
     "spmv_lpr": [4, 8, 16, 32],

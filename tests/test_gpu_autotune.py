@@ -45,3 +45,41 @@ def test_autotune_choices_and_invariance(gpu, tmp_path):
     finally:
         engine.set_tuning("flat_min_n", 32768)
         autotune.reset()
+
+
+def test_stored_tables_keep_the_register_eigensolver(gpu, tmp_path):
+    """Tuning, or a table stored when every chain's launch shape was a knob, leaves chains of up to
+    512 rows on the register kernels: the same pairs bit for bit (the kernels for a basis in memory sum
+    in another order)."""
+    import json
+
+    from impuritymodel_amd import autotune, surrogate
+    from impuritymodel_amd.batched import ground_bases
+    from impuritymodel_amd.engine import Batch, Ops
+
+    fam = surrogate.XASFamily()
+    ms = fam.models(surrogate.sample_params(3, seed=1))
+    ops = Ops([m.hOp for m in ms], [m.restrictions for m in ms], ms[0].n_spin_orbitals)
+    b = Batch(ops, np.arange(len(ms), dtype=np.int32))
+    b.set_seeds(ground_bases(ms, ops.W))
+    b.build(fixed_basis=True)
+
+    def solve():
+        ev, vecs, _, ok = b.eigen(3)
+        assert ok
+        return ev, vecs
+
+    autotune.reset()
+    ev, vecs = solve()
+    p = tmp_path / "t.json"
+    p.write_text(json.dumps({"old": {"eigen_bt": {"best": 512, "ms": {}}, "eigen_wave_max_n": {"best": 1024, "ms": {}}}}))
+    try:
+        assert autotune.load("old", path=str(p))
+        old = solve()
+        autotune.reset()
+        autotune.autotune(eigen_batch=b, repeats=1)
+        tuned = solve()
+    finally:
+        autotune.reset()
+    assert np.array_equal(old[0], ev) and np.array_equal(old[1], vecs)
+    np.testing.assert_allclose(tuned[0], ev, rtol=0, atol=1e-10)  # the check interval may move the last step
