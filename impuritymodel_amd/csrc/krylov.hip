@@ -238,48 +238,6 @@ __device__ __forceinline__ double spmv_t(const int64_t* rowptr, const int32_t* c
   return pa;
 }
 
-// One classical Gram-Schmidt pass of w against V[0..m): coefficients by
-// wave-level dot products, then one update sweep.
-template <int BT, class T>
-__device__ void cgs_pass(const T* V, int m, int64_t n, T* w, double2* coef) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  for (int l = wave; l < m; l += BT / 64) {
-    const T* vl = V + (size_t)l * n;
-    double cx = 0.0, cy = 0.0;
-    for (int64_t i = lane; i < n; i += 64) {
-      const T a = vl[i], b = w[i];
-      cx += re_(a) * re_(b) + im_(a) * im_(b);  // conj(a) * b
-      if constexpr (!is_real_v<T>) cy += re_(a) * im_(b) - im_(a) * re_(b);
-    }
-    cx = wave_sum(cx);
-    if constexpr (!is_real_v<T>) cy = wave_sum(cy);
-    if (lane == 0) coef[l] = make_double2(cx, cy);
-  }
-  __syncthreads();
-  for (int64_t i = threadIdx.x; i < n; i += BT) {
-    double wx = re_(w[i]), wy = im_(w[i]);
-    for (int l = 0; l < m; ++l) {
-      const double2 c = coef[l];
-      const T a = V[(size_t)l * n + i];
-      if constexpr (is_real_v<T>) {
-        wx -= re_(a) * c.x;
-      } else {
-        wx -= re_(a) * c.x - im_(a) * c.y;
-        wy -= re_(a) * c.y + im_(a) * c.x;
-      }
-    }
-    w[i] = mk<T>(wx, wy);
-  }
-  __syncthreads();
-}
-
-template <int BT, class T>
-__device__ __forceinline__ double norm2_t(const T* w, int64_t n, double* red) {
-  double p = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += BT) p += re_(w[i]) * re_(w[i]) + im_(w[i]) * im_(w[i]);
-  return block_sum<BT>(p, red);
-}
-
 // cl[l] = <V_l, w> for l < m (and cl[m] = <w, w> when self), eight vectors
 // per wave at a time so w is read once per eight dot products (and eight
 // loads are in flight together); results in LDS.
@@ -1651,12 +1609,6 @@ __global__ __launch_bounds__(FT) void flat_random_kernel(T* v, int64_t n, uint64
   }
   p = block_sum<FT>(p, red);
   if (threadIdx.x == 0) partial[blockIdx.x] = p;
-}
-
-template <class T>
-__global__ __launch_bounds__(FT) void flat_copy_kernel(const double2* src, T* dst, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * FT + threadIdx.x; i < n; i += (int64_t)gridDim.x * FT)
-    dst[i] = mk<T>(src[i].x, src[i].y);
 }
 
 struct KScratch {

@@ -2,9 +2,9 @@
 // of identical shape, trained and evaluated together (blockIdx.z = member).
 //
 // * gemm_nt_kernel: every GEMM, C[m][n] = sum_k A[m][k] B[n][k] with both
-//   operands k-contiguous and padded to whole tiles: forward (X W^T), input gradient (dZ W, from a transposed copy of W) and weight
-//   gradient (dZ^T X, from transposed copies that the producing epilogues
-//   write).  Epilogues fuse the bias, GELU (pre-activation kept in FP32 for the
+//   operands k-contiguous and padded to whole tiles: forward (X W^T), input
+//   gradient (dZ W, from a transposed copy of W) and weight gradient (dZ^T X,
+//   from transposed copies that the producing epilogues write).  Epilogues fuse the bias, GELU (pre-activation kept in FP32 for the
 //   backward pass), the loss and its gradient, the GELU derivative, the bias
 //   gradients and the Adam update.
 // * gather_kernel, loss_sum_kernel: minibatch inputs and the losses.
@@ -25,7 +25,6 @@ namespace imped {
 
 namespace {
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -36,7 +35,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
 }
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
 // GELU(x) = x Phi(x) and its derivative Phi(x) + x phi(x), Phi(x) = (1 +
 // erf(x / sqrt 2)) / 2 (training: full-precision erf)
@@ -404,11 +402,6 @@ __global__ __launch_bounds__(256) void ensemble_stats_kernel(const float* y, int
     dis[b] = pd / (double)E;
     if (target) l1[b] = pl;
   }
-}
-
-__device__ __forceinline__ double wave_sum64(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
 }
 
 // Sums of NV values over a 256-thread workgroup, broadcast to every thread;
