@@ -19,7 +19,7 @@ namespace {
 // checks (Sturm multisection, inverse iteration on one lane per pair) are a
 // further 20 to 75 us a chain.  Measured on one MI355X, launch time before (basis
 // in LDS or memory, 8 waves per chain) -> now: 4096 complex chains of 90 and 100
-// rows 15.4 -> 4.2 ms, 194 of them 0.53 -> 0.43 ms, 2 of them 0.52 -> 0.41 ms; one
+// rows 15.4 -> 4.1 ms, 194 of them 0.53 -> 0.43 ms, 2 of them 0.52 -> 0.40 ms; one
 // real chain of 190 rows 0.78 -> 0.56 ms.
 template <int NQ, int G, int R, class T>
 __global__ __launch_bounds__(64 * NQ * G, 2) void eigen_reg_kernel(EigenArgs a) {

@@ -21,9 +21,9 @@ namespace {
 // Before, chains beyond 80 KiB of basis kept it in memory (one wave per chain,
 // HBM bound: 3.5 TB/s) and smaller ones in LDS (two chains per CU).  Measured
 // on one MI355X, launch time before -> now: 1728 complex chains of 105..225
-// rows, 150 steps, 29.7 -> 6.9 ms; 60 real chains of up to 733 rows, 150
-// steps, 28.1 -> 2.3 ms; 186 real chains of 30..180 rows, all steps, 11.2 ->
-// 1.2 ms; 18432 complex chains of 60 rows, 60 steps, 6.6 -> 2.5 ms.
+// rows, 150 steps, 29.7 -> 6.0 ms; 60 real chains of up to 733 rows, 150
+// steps, 28.1 -> 2.0 ms; 18432 complex chains of 60 rows, 60 steps, 6.6 -> 2.5 ms;
+// 873 of them 0.38 -> 0.19 ms.
 template <int NQ, int G, int R, class T>
 __global__ __launch_bounds__(64 * NQ * G, 2) void lanczos_reg_kernel(LanczosArgs a) {
   extern __shared__ double2 lds[];

@@ -61,8 +61,8 @@ def _batch(h, v0, K, reorth):
 
 @pytest.mark.parametrize("reorth", [0, 1])
 def test_noalloc_lanczos_equals_batch_entry_point(gpu, reorth):
-    # a 256-thread chain, then smaller one-wave chains on the same scratch
-    # (the last one, with reorthogonalization, keeps its basis in LDS)
+    # a 256-thread chain, then smaller chains on the same scratch (with
+    # reorthogonalization they run on the register kernels)
     for n, K, seed in ((9000, 120, 1), (700, 200, 2), (60, 60, 3)):
         h, v0 = _hermitian(n, seed, 6.0 / n)
         a_ref, b_ref, k_ref, s_ref = _batch(h, v0, K, reorth)
